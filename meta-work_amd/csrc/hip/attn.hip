@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const AttnArgs a) {
     __shared__ float buf[kMaxGroup + 1][D];
     __shared__ float2 cs[D / 2];
     __shared__ double red[4][kMaxGroup + 1];
-    const int pos = *a.npast + t, nk = a.Hkv * D, w = tid >> 6;
+    const int pos = *a.npast + a.t0 + t, nk = a.Hkv * D, w = tid >> 6;
     const bool in = tid < D;
     float v[kMaxGroup + 1];
 #pragma unroll
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void attn_part_kernel(const AttnArgs a) {
     float v[G + 1], vv = 0.f;
     float2 csv = {0.f, 0.f};
     float qnw = 0.f, knw = 0.f;
-    const int npast = *a.npast;
+    const int npast = *a.npast + a.t0;
     if constexpr (F) {
         const bool in = tid < D;
         const int dc = in ? tid : D - 1;
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnArgs a) {
 #pragma unroll
     for (int s = 0; s < 64; s++) pv[s] = part[(int64_t)(s < a.n_split ? s : a.n_split - 1) * (D + 2) + 2 + dc];
     const float gx = a.qg[(int64_t)t * a.qg_s + (int64_t)h * 2 * D + D + dc];   // the output gate
-    const int pos = *a.npast + t, ns = pos / kSplitP + 1;
+    const int pos = *a.npast + a.t0 + t, ns = pos / kSplitP + 1;
     __shared__ float w[64];
     __shared__ float inv_l;
     if (tid < 64) {

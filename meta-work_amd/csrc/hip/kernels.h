@@ -168,6 +168,42 @@ int inc_launch(int32_t *p, int32_t by, hipStream_t st);
 int gemm_max_tokens();
 int gemm_launch(const GemmArgs &a, int64_t part_floats, int n_cnt, hipStream_t st);
 
+// The same products for long prompt pieces (gemm_wide.hip). Activations: one
+// record of kWideRec bytes per 32 tokens and 256-element block (tile-major,
+// then block): for each stage of 64 inner elements the f16 planes hi and lo
+// in MFMA operand order (32 KB in all), then the group sums of hi + lo / 32
+// in two f16 planes (1 KB) and 2^e per token (128 bytes, padded to 1 KB).
+// The token tiles are padded to whole groups of 128 tokens (wide_wq_bytes).
+constexpr int kWideRec = 4 * 8192 + 2048;
+struct WidePrep {
+    const float *x; int32_t xs;
+    const float *x2; int32_t x2s;   // PRO_SWIGLU: up, PRO_GATED_RMS: z
+    int32_t pro;                    // PRO_NONE, PRO_RMSU, PRO_SWIGLU, PRO_GATED_RMS
+    const float *pro_w; float eps; int32_t group;
+    uint8_t *wq;
+    double *ss;                     // PRO_RMSU: sums of x^2 [K/256][T]
+    int32_t K, T;
+    int32_t nb;                     // set by the launch
+};
+struct WideArgs {
+    uint32_t type; int32_t K, T;
+    const uint8_t *wq;
+    int32_t nseg;
+    GemmSeg seg[kGemmMaxSeg];
+    const double *ss; float eps;    // optional: y[t][r] = sum * rms scale of token t (from the sums of x^2)
+    float *part;                    // wide_part_floats() floats
+    int32_t *cnt;                   // wide_counters(rows, T) ints, zero before the first launch, left zero
+    // set by gemm_wide_launch
+    int32_t rt0[kGemmMaxSeg + 1];   // first 32-row tile of each segment (prefix)
+    int32_t nb, nrg, G;             // blocks per row, row groups, work-groups
+    int64_t P;                      // units
+};
+size_t wide_wq_bytes(int K, int T);
+int64_t wide_part_floats();
+int wide_counters(int64_t rows, int T);   // rows in all segments of a launch
+int wide_prep_launch(const WidePrep &a, hipStream_t st);
+int gemm_wide_launch(const WideArgs &a, int64_t part_floats, int n_cnt, hipStream_t st);
+
 // Repack a GGUF tensor into the device layout. dst must hold `bytes` =
 // n_rows * row_bytes(type, k); src is host memory in GGUF layout.
 int upload_repack(uint32_t type, const void *src, int64_t n_rows, int64_t k, uint8_t *dst,
@@ -189,6 +225,7 @@ struct AttnArgs {
     int32_t T, H, Hkv, D, n_rot, n_ctx, n_split;
     float eps, scale;
     uint8_t *xq;                         // optional: prepared activations of out (no prologue)
+    int32_t t0;                          // token 0 sits at position *npast + t0
 };
 int attn_launch(const AttnArgs &a, hipStream_t st);
 int attn_splits(int n_ctx);             // 64-position splits covering n_ctx

@@ -37,6 +37,21 @@ namespace {
 constexpr int kSnapSlots = 9;       // 0..7 for callers, kDecodeSlot for xjh_chain_decode
 constexpr int kDecodeSlot = kSnapSlots - 1;
 
+// Buffers of the wide GEMM (gemm_wide.hip): activation records, an RMSNorm
+// input's sums of x^2, partial tiles and arrival counters (zero between launches).
+struct WideBuf {
+    uint8_t *wq = nullptr;
+    double *ss = nullptr;
+    float *part = nullptr;
+    int64_t part_floats = 0;
+    int32_t *cnt = nullptr;
+    int32_t n_cnt = 0;
+};
+
+// Chunks of at least kGemmMinT tokens take the matrix-core GEMM and the
+// chunked delta rule.
+constexpr int kGemmMinT = 16;
+
 struct HLayer {
     bool rec = false;
     const float *attn_norm = nullptr, *post_norm = nullptr;
@@ -84,6 +99,8 @@ struct HStage {
     int64_t gpart_floats = 0;
     int32_t *gcnt = nullptr;   // the GEMM's arrival counters (zero between launches)
     int32_t n_gcnt = 0;
+    WideBuf wide;              // buffers of the wide GEMM (max_batch > 64)
+    int gemm_min = kGemmMinT;  // tokens from which a chunk takes the matrix-core path
     float2 *rope = nullptr;
     float *h_x = nullptr;            // pinned staging [max_batch][n_embd]
     int32_t *h_i = nullptr;          // pinned scalar
@@ -186,8 +203,9 @@ struct Gemv {
     bool prepared = false;
     explicit Gemv(uint8_t *xq, Profile *p = nullptr) : prof(p) { a.xq = xq; }
     Gemv(uint8_t *xq, Profile *p, float *tsc_, float *part_, int64_t part_floats_, int32_t *cnt_, int32_t n_cnt_,
-         uint8_t *hq_)
-        : prof(p), tsc(tsc_), part(part_), part_floats(part_floats_), cnt(cnt_), n_cnt(n_cnt_), hq(hq_) {
+         uint8_t *hq_, const WideBuf *wide_, int gemm_min_)
+        : prof(p), tsc(tsc_), part(part_), part_floats(part_floats_), cnt(cnt_), n_cnt(n_cnt_), hq(hq_), wide(wide_),
+          gemm_min(gemm_min_) {
         a.xq = xq;
     }
     Gemv &seg(const DevW &w, float *y, int ys, int epi) {
@@ -243,16 +261,17 @@ struct Gemv {
     uint8_t *hq = nullptr;
     bool hq_ready = false;
     bool hq_out = false;   // set by a GEMM run whose SwiGLU prep built the next input's hq
+    const WideBuf *wide = nullptr;
+    int gemm_min = kGemmMinT;
     // Chunks of at least kGemmMinT tokens take the matrix-core GEMM
     // (gemm.hip): the prep launch builds the T tokens' activations once, the
     // RMSNorm scale is applied per token after the dot products (as the GEMV
     // applies it), the conv + SiLU runs as its own launch and the SwiGLU tail
     // as the down projection's prep. Segments the GEMM does not take (float
     // rows) and every other case keep the GEMV.
-    static constexpr int kGemmMinT = 16;
     bool gemm_ok(int T) const {
         static const bool on = env_int("XJ_PREFILL_GEMM", 1) != 0;
-        if (!on || T < kGemmMinT || prof || !tsc || !part || !cnt || !a.xq || !hq) return false;
+        if (!on || T < gemm_min || prof || !tsc || !part || !cnt || !a.xq || !hq) return false;
         if (a.pro != PRO_NONE && a.pro != PRO_RMSU && a.pro != PRO_SWIGLU && a.pro != PRO_GATED_RMS) return false;
         if (a.post.mode != POST_NONE && a.post.mode != POST_SWIGLU) return false;
         if (a.K % 256) return false;
@@ -260,9 +279,48 @@ struct Gemv {
         for (int i = 0; i < a.nseg; i++) any = any || a.seg[i].type == XJ_Q4_K || a.seg[i].type == XJ_Q6_K;
         return any;
     }
+    // Chunks beyond the 64 tokens of a gemm.hip launch take the wide GEMM
+    // (gemm_wide.hip; 18432 x 2560 Q4_K, T = 128: 45 us against two launches of
+    // 37 us, T = 1024: 232 us against 16), which reads the plain input: a
+    // caller whose input would be prepared asks first and passes x instead.
+    bool wide_ok(int T) const {
+        auto al = [](const void *p, int32_t s) { return !((uintptr_t)p & 15) && !(s & 3); };
+        if (T <= gemm_max_tokens() || !gemm_ok(T) || prepared || !wide || !wide->wq || !a.x || !al(a.x, a.xs)) return false;
+        const bool two = a.pro == PRO_SWIGLU || a.pro == PRO_GATED_RMS;
+        if (two && (!a.x2 || !al(a.x2, a.x2s))) return false;
+        if ((a.pro == PRO_RMSU || a.pro == PRO_GATED_RMS) && !al(a.pro_w, 0)) return false;
+        return a.pro != PRO_GATED_RMS || a.group == 64 || a.group == 128;
+    }
+    int wide_gemm(int T, hipStream_t st) {
+        WidePrep p{};
+        p.x = a.x; p.xs = a.xs; p.x2 = a.x2; p.x2s = a.x2s; p.pro = a.pro; p.pro_w = a.pro_w; p.eps = a.eps; p.group = a.group;
+        p.wq = wide->wq; p.ss = wide->ss; p.K = a.K; p.T = T;
+        if (wide_prep_launch(p, st)) return -1;
+        for (uint32_t ty : {XJ_Q4_K, XJ_Q6_K}) {
+            WideArgs g{};
+            g.type = ty; g.K = a.K; g.T = T; g.wq = wide->wq; g.part = wide->part; g.cnt = wide->cnt;
+            if (a.pro == PRO_RMSU) g.ss = wide->ss, g.eps = a.eps;
+            for (int i = 0; i < a.nseg; i++) {
+                const GSeg &s = a.seg[i];
+                if (s.type == ty) g.seg[g.nseg++] = GemmSeg{s.w, s.n_rows, s.y, s.ys, s.epi == EPI_ADD};
+            }
+            if (g.nseg && gemm_wide_launch(g, wide->part_floats, wide->n_cnt, st)) return -1;
+        }
+        // segments of other types run on the GEMV, which reads the prep kernel's digits
+        for (int i = 0; i < a.nseg; i++)
+            if (a.seg[i].type != XJ_Q4_K && a.seg[i].type != XJ_Q6_K) {
+                GArgs b = a;
+                b.T = T;
+                return prep_launch(b, st);
+            }
+        return 0;
+    }
     int run_gemm(int T, hipStream_t st) {
         const int64_t xs = xq_off(a.K).stride, hs = hq_stride(a.K);
-        if (!prepared) {   // the T tokens' activations, once (no digits when no segment takes the GEMV)
+        const bool w = wide_ok(T);
+        if (w) {
+            if (wide_gemm(T, st)) return -1;
+        } else if (!prepared) {   // the T tokens' activations, once (no digits when no segment takes the GEMV)
             GArgs b = a;
             b.T = T;
             b.hq = hq;
@@ -274,7 +332,7 @@ struct Gemv {
             return -1;
         }
         const bool rms = a.pro == PRO_RMSU;
-        if (rms && rms_scale_launch(a.xq, xs, a.K, T, a.eps, tsc, st)) return -1;
+        if (!w && rms && rms_scale_launch(a.xq, xs, a.K, T, a.eps, tsc, st)) return -1;
         const int mt = gemm_max_tokens(), tile = gemv_max_tile(a.K);
         // the Q4_K and Q6_K segments in one launch sharing the activations,
         // each type on its own share of the work-groups (an attention
@@ -302,7 +360,9 @@ struct Gemv {
                 if (s.type == ty) g.seg[g.nseg++] = GemmSeg{s.w, s.n_rows, s.y, s.ys, s.epi == EPI_ADD};
             }
         }
-        if (mixed_on && gk[0].nseg && gk[1].nseg) {
+        if (w) {
+            // every K-quant segment is done
+        } else if (mixed_on && gk[0].nseg && gk[1].nseg) {
             GemmArgs g = gk[0];
             for (int i = 0; i < gk[1].nseg; i++) g.seg[g.nseg++] = gk[1].seg[i];
             g.n6 = gk[1].nseg;
@@ -397,6 +457,8 @@ struct Gemv {
 
 // --------------------------------------------------------------- layers --
 
+constexpr int kAttnT = 64;   // tokens per attention launch of a long piece
+
 // Layer il on T tokens of x. The GEMVs that read the residual stream build
 // their RMSNorm activations inside their own work-groups; every other
 // prologue is produced by the kernel before its GEMV: the down input by
@@ -406,7 +468,7 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
     HLayer &L = S->L[il - S->s.l0];
     const int E = hp.n_embd, FF = hp.n_ff;
     // every GEMV of the layer with the stage's prefill buffers
-    auto gemv = [&](uint8_t *xq) { return Gemv(xq, pf, S->tsc, S->gpart, S->gpart_floats, S->gcnt, S->n_gcnt, S->hq); };
+    auto gemv = [&](uint8_t *xq) { return Gemv(xq, pf, S->tsc, S->gpart, S->gpart_floats, S->gcnt, S->n_gcnt, S->hq, &S->wide, S->gemm_min); };
     auto rms_in = [&](Gemv &g, const float *w) {
         g.a.x = x; g.a.xs = E; g.a.pro = PRO_RMSU; g.a.pro_w = w; g.a.eps = hp.eps;
     };
@@ -425,7 +487,7 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
         // then the gated RMSNorm (xj_cpu.c:215-217) as ssm_out's prep launch
         static const bool chunked_on = env_int("XJ_PREFILL_CHUNKED", 1) != 0;
         const int Sd = hp.s_k;
-        if (chunked_on && !pf && keep_n == 0 && T >= Gemv::kGemmMinT && S->dwork && (Sd == 64 || Sd == 128) &&
+        if (chunked_on && !pf && keep_n == 0 && T >= S->gemm_min && S->dwork && (Sd == 64 || Sd == 128) &&
             hp.s_v == Sd && T <= S->s.max_batch) {
             DeltaPrepArgs dp{};
             dp.qkv = S->qkv; dp.qkv_s = CD; dp.k_off = hp.key_dim; dp.v_off = 2 * hp.key_dim;
@@ -484,11 +546,21 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
         at.T = T; at.H = Hq; at.Hkv = Hkv; at.D = D; at.n_rot = hp.n_rot; at.n_ctx = S->s.n_ctx;
         at.n_split = attn_splits(S->s.n_ctx);
         at.eps = hp.eps; at.scale = 1.0f / sqrtf((float)D);
-        at.xq = S->xq_att;
-        if (!pf && attn_launch(at, st)) return -1;
         Gemv q = gemv(S->xq_att);
-        q.prepared = true;
+        q.a.x = S->o; q.a.xs = Hq * D; q.a.pro = PRO_NONE;
         q.seg(L.wo, x, E, EPI_ADD);
+        q.prepared = !q.wide_ok(T);
+        if (q.prepared) q.a.x = nullptr;
+        // long pieces in slices of 64 tokens (the split partials' scratch)
+        for (int t0 = 0; !pf && t0 < T; t0 += kAttnT) {
+            AttnArgs b = at;
+            b.t0 = t0;
+            b.T = T - t0 < kAttnT ? T - t0 : kAttnT;
+            b.qg += (int64_t)t0 * at.qg_s; b.kn += (int64_t)t0 * at.kn_s; b.vn += (int64_t)t0 * at.vn_s;
+            b.out += (int64_t)t0 * Hq * D;
+            b.xq = q.prepared ? S->xq_att + (int64_t)t0 * xq_off(Hq * D).stride : nullptr;
+            if (attn_launch(b, st)) return -1;
+        }
         if (q.run(T, st)) return -1;
     }
     Gemv f = gemv(S->xq_e);
@@ -499,30 +571,31 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
     // down read a prepared xq instead)
     const uint32_t dt = L.ffn_down.type;
     const bool h = T == 1 && dt != XJ_F32 && dt != XJ_F16 && dt != XJ_BF16 && f.swiglu_h(S->g);
-    if (!h) f.post(POST_SWIGLU, S->xq_ff, S->cnt_grp);
-    if (f.run(T, st)) return -1;
     Gemv dn = gemv(S->xq_ff);
-    if (h) {
+    dn.a.x = S->g; dn.a.xs = FF; dn.a.x2 = S->u; dn.a.x2s = FF; dn.a.pro = PRO_SWIGLU;
+    dn.seg(L.ffn_down, x, E, EPI_ADD);
+    const bool wide = f.wide_ok(T) && dn.wide_ok(T);   // silu(gate) * up formed by down's own prep
+    if (!h && !wide) f.post(POST_SWIGLU, S->xq_ff, S->cnt_grp);
+    if (f.run(T, st)) return -1;
+    if (!wide) dn.a.x = dn.a.x2 = nullptr, dn.a.pro = PRO_NONE;
+    if (wide) {
+        // a.x, a.x2 set above
+    } else if (h) {
         dn.a.x = S->g; dn.a.xs = FF; dn.a.pro = PRO_X;
     } else {
         dn.prepared = true;
         dn.hq_ready = f.hq_out;
     }
     dn.a.inc_ptr = inc; dn.a.inc_by = T;
-    dn.seg(L.ffn_down, x, E, EPI_ADD);
     return dn.run(T, st);
 }
 
-// Layers [lo, hi) of the stage; inc: the stage's position counter advances
-// by T after the last of them.
-int enqueue_layer_range(HStage *S, int lo, int hi, float *x, int T, int keep_n, bool inc, hipStream_t st,
-                        Profile *pf = nullptr) {
-    for (int il = lo; il < hi; il++)
-        if (enqueue_layer(S, il, x, T, keep_n, inc && il + 1 == hi ? S->npast : nullptr, st, pf)) return -1;
-    return 0;
-}
+// Every layer of the stage; inc: the stage's position counter advances by T
+// after the last of them.
 int enqueue_layers(HStage *S, float *x, int T, int keep_n, bool inc, hipStream_t st, Profile *pf = nullptr) {
-    return enqueue_layer_range(S, S->s.l0, S->s.l1, x, T, keep_n, inc, st, pf);
+    for (int il = S->s.l0; il < S->s.l1; il++)
+        if (enqueue_layer(S, il, x, T, keep_n, inc && il + 1 == S->s.l1 ? S->npast : nullptr, st, pf)) return -1;
+    return 0;
 }
 
 // logits[t] = output . rmsnorm(x[t]) * output_norm; greedy partial keys into S->amax
@@ -743,7 +816,7 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
     S->g = dalloc<float>(S, mb * sf, err, errlen);
     S->u = dalloc<float>(S, mb * sf, err, errlen);
     S->qr = dalloc<float>(S, mb * hp.n_head * (size_t)hp.head_dim, err, errlen);
-    S->scores = dalloc<float>(S, mb * hp.n_head * (size_t)attn_splits(n_ctx) * (hp.head_dim + 2), err, errlen);
+    S->scores = dalloc<float>(S, (mb < kAttnT ? mb : kAttnT) * hp.n_head * (size_t)attn_splits(n_ctx) * (hp.head_dim + 2), err, errlen);
     S->npast = dalloc<int32_t>(S, 1, err, errlen);
     // prefill on the matrix cores (chunks of at least 16 tokens)
     S->tsc = dalloc<float>(S, mb, err, errlen);
@@ -756,6 +829,17 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
     S->hq = dalloc<uint8_t>(S, mb * (size_t)hq_stride((int)sf), err, errlen);
     if (!S->tsc || !S->gpart || !S->gcnt || !S->hq) return false;
     XJ_CHECK(hipMemset(S->gcnt, 0, (size_t)S->n_gcnt * 4), err, errlen, false);
+    if ((int)mb > gemm_max_tokens()) {
+        WideBuf &w = S->wide;
+        w.wq = dalloc<uint8_t>(S, wide_wq_bytes((int)(sf / 256 * 256), (int)mb), err, errlen);
+        w.ss = dalloc<double>(S, mb * (E / 256), err, errlen);
+        w.part_floats = wide_part_floats();
+        w.part = dalloc<float>(S, (size_t)w.part_floats, err, errlen);
+        w.n_cnt = wide_counters(grows, (int)mb);
+        w.cnt = dalloc<int32_t>(S, (size_t)w.n_cnt, err, errlen);
+        if (!w.wq || !w.ss || !w.part || !w.cnt) return false;
+        XJ_CHECK(hipMemset(w.cnt, 0, (size_t)w.n_cnt * 4), err, errlen, false);
+    }
     {
         bool rec = false;
         for (int il = S->s.l0; il < S->s.l1 && il < hp.n_layer; il++) rec = rec || S->s.m->layers[il].recurrent;
@@ -783,38 +867,27 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
     return true;
 }
 
-// A second set of scratch for a stage whose prompt chunks run as two
-// pipelined halves (chain_eval): the stage's weights, layer states and head
-// buffers shared, its own scratch, stream and position counter.
-static HStage *twin_new(HStage *S, char *err, size_t errlen) {
+// A second set of scratch, for pieces of a prompt longer than the stage's
+// max_batch (chain_eval): the stage's weights, layer states, stream and
+// position counter.
+static HStage *twin_new(HStage *S, int max_batch, char *err, size_t errlen) {
     HStage *T = new HStage();
     T->s = S->s;
-    T->L = S->L;
-    T->output = S->output; T->tok_embd = S->tok_embd; T->out_norm = S->out_norm;
-    T->rope = S->rope; T->logits = S->logits; T->amax = S->amax;
-    T->head_nwg = S->head_nwg; T->head_rows = S->head_rows;
-    T->conv_n = S->conv_n; T->ssm_n = S->ssm_n; T->n_ck = S->n_ck;
-    if (hipStreamCreateWithFlags(&T->st, hipStreamNonBlocking) != hipSuccess) {
-        snprintf(err, errlen, "stream creation failed");
-        T->st = nullptr;
-    } else if (hipHostMalloc((void **)&T->h_i, 64, hipHostMallocDefault) != hipSuccess) {
-        snprintf(err, errlen, "pinned allocation failed");
-        T->h_i = nullptr;
-    } else if (alloc_scratch(T, err, errlen)) {
-        return T;
+    T->s.max_batch = max_batch;
+    T->st = S->st;
+    T->rope = S->rope;
+    T->conv_n = S->conv_n; T->ssm_n = S->ssm_n;
+    if (!alloc_scratch(T, err, errlen)) {
+        for (void *p : T->allocs) (void)hipFree(p);
+        delete T;
+        return nullptr;
     }
-    for (void *p : T->allocs) (void)hipFree(p);
-    if (T->h_i) (void)hipHostFree(T->h_i);
-    if (T->st) (void)hipStreamDestroy(T->st);
-    delete T;
-    return nullptr;
+    T->npast = S->npast;
+    return T;
 }
 static void twin_free(HStage *T) {
     if (!T) return;
-    if (T->st) (void)hipStreamSynchronize(T->st);
     for (void *p : T->allocs) (void)hipFree(p);
-    if (T->h_i) (void)hipHostFree(T->h_i);
-    if (T->st) (void)hipStreamDestroy(T->st);
     delete T;
 }
 
@@ -865,11 +938,14 @@ extern "C" uint64_t xj_hip_stage_state_bytes(const xj_model *m, int l0, int l1, 
             b += 2ull * 2 * n_ctx * hp.n_head_kv * hp.head_dim;
     }
     b += 10ull * 4 * max_batch * scratch_floats(hp) +
-         4ull * max_batch * hp.n_head * ((n_ctx + 63) / 64) * (hp.head_dim + 2);
+         4ull * (max_batch < kAttnT ? max_batch : kAttnT) * hp.n_head * ((n_ctx + 63) / 64) * (hp.head_dim + 2);
     // prefill on the matrix cores: RMSNorm scales, K-split partials and counters, chunked-rule work
     const int64_t grows = 2 * (int64_t)scratch_floats(hp) + 2 * (int64_t)hp.h_v;
     b += 4ull * max_batch + 4ull * gemm_part_floats(grows, max_batch < gemm_max_tokens() ? max_batch : gemm_max_tokens()) +
          4ull * gemm_counters(grows) + (uint64_t)max_batch * hq_stride((int)scratch_floats(hp));
+    if (max_batch > gemm_max_tokens())
+        b += wide_wq_bytes((int)(scratch_floats(hp) / 256 * 256), max_batch) + 8ull * max_batch * (hp.n_embd / 256) +
+             4ull * wide_part_floats() + 4ull * wide_counters(grows, max_batch);
     bool rec = false;
     for (int il = l0; il < l1 && il < (int)hp.n_layer; il++) rec = rec || m->layers[il].recurrent;
     if (rec) b += delta_chunked_work_bytes(hp.h_v, hp.s_k, max_batch, 64);
@@ -1097,10 +1173,14 @@ extern "C" int xj_hip_stage_restore(xj_stage *s, int slot, int n_past, char *err
 
 // ================================================================= chain ==
 
-constexpr int kMaxParts = 4;   // parts of a single stage's layers in a pipelined prefill
+// Tokens of a prompt that go through a layer at once, whatever max_batch is:
+// a weight is decoded once per 128 tokens, and every launch fills the chip.
+// Stages whose max_batch is above half of it run their own chunks.
+constexpr int kPieceT = 1024;
 struct xjh_chain {
     std::vector<HStage *> st;
-    std::vector<HStage *> twins;   // a single stage's later parts of the layers in prefill (twin_new)
+    std::vector<HStage *> twins;   // per stage, scratch for prompt pieces of up to piece tokens (twin_new)
+    int piece = 0;
     hipStream_t stream = nullptr;
     float *x = nullptr;
     int mb = 0, hist_cap = 0;
@@ -1128,23 +1208,26 @@ struct xjh_chain {
     hipGraph_t graph_s = nullptr;
 };
 
-// Parts of a single stage's layers in a prompt of several chunks
-// (XJ_STAGE_SPLIT, with chunks overlapped on the parts' streams), else 1.
-static int stage_parts(const xjh_chain *c) {
-    static const bool overlap = env_int("XJ_CHAIN_OVERLAP", 1) != 0;
-    static const int split_env = env_int("XJ_STAGE_SPLIT", 3);
-    if (c->st.size() != 1 || !overlap) return 1;
-    const int nl = c->st[0]->s.l1 - c->st[0]->s.l0;
-    return split_env < 1 ? 1 : split_env > kMaxParts ? kMaxParts : split_env > nl ? nl : split_env;
-}
-// the later parts' scratch sets (twin_new), created once
-static int chain_twins(xjh_chain *c, int npart, char *err, size_t errlen) {
-    while ((int)c->twins.size() < npart - 1) {
-        HStage *T = twin_new(c->st[0], err, errlen);
-        if (!T) return -1;
+// Every stage's scratch for prompt pieces, created once; false: none (max_batch
+// too large to need it, or no memory: prompts then run in chunks of max_batch).
+static bool chain_twins(xjh_chain *c) {
+    static const bool on = env_int("XJ_PREFILL_GEMM", 1) != 0;
+    if (!on || c->mb > kPieceT / 2 || c->piece < 0) return false;
+    if (c->piece > 0) return true;
+    char err[256];
+    const int n_ctx = (c->st[0]->s.n_ctx + 127) / 128 * 128;
+    for (auto *S : c->st) {
+        HStage *T = twin_new(S, n_ctx < kPieceT ? n_ctx : kPieceT, err, sizeof err);
+        if (!T) {
+            for (HStage *t : c->twins) twin_free(t);
+            c->twins.clear();
+            c->piece = -1;
+            return false;
+        }
         c->twins.push_back(T);
     }
-    return 0;
+    c->piece = c->twins[0]->s.max_batch;
+    return true;
 }
 extern "C" void xjh_chain_free(xjh_chain *c) {
     if (!c) return;
@@ -1199,7 +1282,7 @@ extern "C" xjh_chain *xjh_chain_new(xj_stage **stages, int n, char *err, size_t 
         xjh_chain_free(c);
         return nullptr;
     }
-    const size_t nev = c->st.size() < kMaxParts ? kMaxParts : c->st.size();   // a single stage may run in parts
+    const size_t nev = c->st.size();
     c->ev_done.assign(nev, nullptr);
     c->ev_taken.assign(nev, nullptr);
     for (size_t i = 0; i < nev; i++)
@@ -1209,13 +1292,9 @@ extern "C" xjh_chain *xjh_chain_new(xj_stage **stages, int n, char *err, size_t 
             xjh_chain_free(c);
             return nullptr;
         }
-    // a stage whose chunks take the prefill GEMM gets its parts' scratch now,
-    // so that its first long prompt does not pay for the allocations
-    // (a 4B 1024-token prefill: 0.083 s on the first call, 0.073 s after)
-    if (c->mb >= Gemv::kGemmMinT && stage_parts(c) > 1 && chain_twins(c, stage_parts(c), err, errlen)) {
-        xjh_chain_free(c);
-        return nullptr;
-    }
+    // stages whose chunks take the prefill GEMM get the pieces' scratch now, so
+    // that the first long prompt does not pay for the allocations
+    if (c->mb >= kGemmMinT) (void)chain_twins(c);
     return c;
 }
 
@@ -1226,128 +1305,124 @@ static int chain_sync(xjh_chain *c, char *err, size_t errlen) {
     return 0;
 }
 
-// The prompt in chunks of max_batch, the stages pipelined (pipe/core/xj_net.c:561-604
-// pipelines a remote worker's half against the host's): each stage runs on its
-// own stream from its own hidden-state buffer, so stage i works on chunk k + 1
-// while stage i + 1 works on chunk k. A single stage's layers run the same
-// way in XJ_STAGE_SPLIT parts (3: a 4B 1024-token prefill 0.118 -> 0.083 s;
-// 2 parts 0.091 s, 4 parts 0.093 s). Stage i + 1 takes chunk k by a device
-// copy once stage i has finished it (event done[i]); stage i overwrites its
-// buffer with chunk k + 1 only after that copy (event taken[i + 1]). Every
-// stage's n_past advances on the device at the end of each chunk, so no host
-// round trip separates the chunks; XJ_CHAIN_OVERLAP=0 runs all stages on one
-// stream.
+// A prompt longer than max_batch, in pieces: of up to kPieceT tokens on the
+// stages' second scratch (chain_twins; from the 16 tokens on that take the
+// GEMM), else in chunks of max_batch. The stages are pipelined
+// (pipe/core/xj_net.c:561-604 pipelines a remote worker's half against the
+// host's): each stage runs on its own stream from its own hidden-state buffer,
+// so stage i works on piece k + 1 while stage i + 1 works on piece k. Stage
+// i + 1 takes piece k by a device copy once stage i has finished it (event
+// done[i]); stage i overwrites its buffer with piece k + 1 only after that copy
+// (event taken[i + 1]). Every stage's n_past advances on the device at the end
+// of each piece, so no host round trip separates them; XJ_CHAIN_OVERLAP=0 runs
+// all stages on one stream.
 static int chain_finish(xjh_chain *c, int nl, int32_t *argmax, char *err, size_t errlen);
 // wait = false: returns once everything is enqueued (nlog > 0, no logits);
 // chain_finish collects the argmax of the nlog rows.
 static int chain_eval(xjh_chain *c, const int32_t *tokens, int n, int nlog, int keep, float *logits, int32_t *argmax,
                       char *err, size_t errlen, bool wait = true) {
-    const int B = c->mb, E = c->st[0]->s.m->hp.n_embd, ns = (int)c->st.size();
+    const int B = c->mb, E = c->st[0]->s.m->hp.n_embd, np = (int)c->st.size();
     if (!wait && (nlog < 1 || logits || n > B)) { snprintf(err, errlen, "asynchronous eval of one chunk with argmax only"); return -1; }
     if (n <= 0) { snprintf(err, errlen, "no tokens"); return -1; }
     if (keep && n > B) { snprintf(err, errlen, "verify batch %d exceeds max_batch %d", n, B); return -1; }
     static const bool overlap = env_int("XJ_CHAIN_OVERLAP", 1) != 0;
-    // the pipeline's parts: every stage, or a single stage's layers in
-    // XJ_STAGE_SPLIT contiguous parts (the later ones on twins' scratch and
-    // streams) when the prompt spans several chunks
-    struct Part { HStage *S; int lo, hi; bool twin; };
-    std::vector<Part> parts;
-    HStage *S0 = c->st[0];
-    const int nl = S0->s.l1 - S0->s.l0;
-    const int npart = stage_parts(c);
-    if (npart > 1 && n > B && !keep) {
-        if (chain_twins(c, npart, err, errlen)) return -1;
-        for (int p = 0; p < npart; p++) {
-            HStage *S = p ? c->twins[p - 1] : S0;
-            if (p) {
-                S->L = S0->L;   // checkpoint and snapshot buffers allocated since
-                S->n_ck = S0->n_ck;
-            }
-            parts.push_back(Part{S, S0->s.l0 + nl * p / npart, S0->s.l0 + nl * (p + 1) / npart, p > 0});
-        }
-    } else {
-        for (auto *S : c->st) parts.push_back(Part{S, S->s.l0, S->s.l1, false});
-    }
-    const int np = (int)parts.size();
-    HStage *head = parts.back().S;
-    auto stream_of = [&](int i) { return overlap ? parts[i].S->st : c->stream; };
+    HStage *head = c->st.back();
+    auto stream_of = [&](int i) { return overlap ? c->st[i]->st : c->stream; };
     auto fail_sync = [&]() {
-        for (int i = 0; i < np; i++) (void)hipStreamSynchronize(parts[i].S->st);
+        for (int i = 0; i < np; i++) (void)hipStreamSynchronize(stream_of(i));
         for (auto *S : c->st) S->s.keep = 0;
         return -1;
     };
     for (auto *S : c->st)
         if (S->s.n_past + n > S->s.n_ctx) { snprintf(err, errlen, "context full (%d)", S->s.n_ctx); return -1; }
+    const bool wide = n > B && n >= kGemmMinT && chain_twins(c);
+    // stages whose own chunks are too short for the matrix cores (max_batch <
+    // 16) keep the GEMV's arithmetic for prompts up to twice that length, bit
+    // for bit that of the same tokens in chunks or steps
+    const int gemm_min = B < kGemmMinT && n < 2 * kGemmMinT ? 2 * kGemmMinT : kGemmMinT;
     if (n > c->prompt_cap) {
         if (c->d_prompt) (void)hipFree(c->d_prompt);
         c->d_prompt = nullptr, c->prompt_cap = 0;
         if (hipMalloc(&c->d_prompt, 4 * (size_t)n) != hipSuccess) { snprintf(err, errlen, "prompt allocation failed"); return -1; }
         c->prompt_cap = n;
     }
-    // the ids (synchronous copy from the caller's memory) and every part's
-    // starting position (a twin starts where its stage is)
+    // the ids (synchronous copy from the caller's memory) and every stage's
+    // starting position
     if (hipMemcpy(c->d_prompt, tokens, 4 * (size_t)n, hipMemcpyHostToDevice) != hipSuccess) {
         snprintf(err, errlen, "token upload failed"); return -1;
     }
     for (int i = 0; i < np; i++) {
-        HStage *S = parts[i].S;
-        *S->h_i = parts[i].twin ? S0->s.n_past : S->s.n_past;
+        HStage *S = c->st[i];
+        *S->h_i = S->s.n_past;
         if (hipMemcpyAsync(S->npast, S->h_i, 4, hipMemcpyHostToDevice, stream_of(i)) != hipSuccess ||
             hipStreamSynchronize(stream_of(i)) != hipSuccess) {   // h_i is reused by later calls
             snprintf(err, errlen, "position upload failed"); return -1;
         }
     }
-    for (int k0 = 0; k0 < n; k0 += B) {
-        const int T = n - k0 < B ? n - k0 : B;
+    auto x_of = [&](int i) { return wide ? c->twins[i]->x : c->st[i]->x; };
+    int Tp = 0;   // tokens of the last piece
+    for (int k0 = 0; k0 < n; k0 += Tp) {
+        const int left = n - k0;
+        if (!wide) Tp = left < B ? left : B;
+        // the last piece keeps at least max_batch tokens (the rows a caller may ask for)
+        else Tp = left <= c->piece ? left : left - c->piece < B ? c->piece / 2 : c->piece;
         for (int i = 0; i < np; i++) {
-            HStage *S = parts[i].S;
+            HStage *S = c->st[i];
             hipStream_t st = stream_of(i);
+            float *x = x_of(i);
             if (i == 0) {
-                // chunk k0 into part 0's buffer, once part 1 has taken the previous chunk
+                // piece k0 into stage 0's buffer, once stage 1 has taken the previous one
                 if (np > 1 && k0 > 0 && hipStreamWaitEvent(st, c->ev_taken[1], 0) != hipSuccess) return fail_sync();
-                EmbedArgs ea{c->d_prompt + k0, S->tok_embd, S->x, T};
+                EmbedArgs ea{c->d_prompt + k0, S->tok_embd, x, Tp};
                 if (embed_launch(ea, st)) { snprintf(err, errlen, "embed launch failed"); return fail_sync(); }
             } else {
-                // this part's previous chunk is done with its buffer (same stream); the
-                // upstream part's output of this chunk is final
+                // this stage's previous piece is done with its buffer (same stream); the
+                // upstream stage's output of this piece is final
                 if (i + 1 < np && k0 > 0 && hipStreamWaitEvent(st, c->ev_taken[i + 1], 0) != hipSuccess) return fail_sync();
                 if (hipStreamWaitEvent(st, c->ev_done[i - 1], 0) != hipSuccess ||
-                    hipMemcpyAsync(S->x, parts[i - 1].S->x, sizeof(float) * (size_t)T * E, hipMemcpyDeviceToDevice, st) != hipSuccess ||
+                    hipMemcpyAsync(x, x_of(i - 1), sizeof(float) * (size_t)Tp * E, hipMemcpyDeviceToDevice, st) != hipSuccess ||
                     hipEventRecord(c->ev_taken[i], st) != hipSuccess) {
                     snprintf(err, errlen, "chunk hand-off failed"); return fail_sync();
                 }
             }
             int keep_n = 0;
-            if (!parts[i].twin) {
-                if (keep) S->s.keep = T;
-                if (begin_forward(S, T, &keep_n, err, errlen)) return fail_sync();
+            HStage *R = S;   // the scratch the layers run on
+            if (wide) {
+                if (reset_check(S, err, errlen)) return fail_sync();
+                R = c->twins[i];
+                R->L = S->L;   // checkpoint and snapshot buffers allocated since
+                R->gemm_min = gemm_min;
+                S->s.keep = 0;
+                S->s.ck_start = S->s.n_past;
+                S->s.ck_T = 0;
+            } else {
+                if (keep) S->s.keep = Tp;
+                if (begin_forward(S, Tp, &keep_n, err, errlen)) return fail_sync();
             }
-            if (enqueue_layer_range(S, parts[i].lo, parts[i].hi, S->x, T, keep_n, true, st) ||
-                hipEventRecord(c->ev_done[i], st) != hipSuccess) {
+            if (enqueue_layers(R, x, Tp, keep_n, true, st) || hipEventRecord(c->ev_done[i], st) != hipSuccess) {
                 snprintf(err, errlen, "layer launch failed"); return fail_sync();
             }
-            if (!parts[i].twin) {
-                S->s.n_past += T;
-                if (k0 + T < n) S->s.keep = 0;
-            }
+            S->s.n_past += Tp;
+            if (k0 + Tp < n) S->s.keep = 0;
         }
     }
-    const int T = n - (n - 1) / B * B;   // tokens of the last chunk
+    const int T = n - (n - 1) / B * B;   // tokens of the last chunk of max_batch, the piece's last rows
+    const float *xl = x_of(np - 1) + (int64_t)(Tp - T) * E;
     hipStream_t hs = stream_of(np - 1);
     if (nlog > 0) {
         const int nl = nlog < T ? nlog : T;
-        if (enqueue_head(head, head->x + (int64_t)(T - nl) * E, nl, head->logits, hs) ||
+        if (enqueue_head(head, xl + (int64_t)(T - nl) * E, nl, head->logits, hs) ||
             argmax_finalize_launch(head->amax, head->head_nwg, nl, c->d_argmax, c->d_tok, nullptr, nullptr, hs)) {
             snprintf(err, errlen, "head launch failed"); return fail_sync();
         }
     }
     // the last chunk's hidden rows where the decode step and the drivers read
     // them (the chain's buffer, stage 0's); the head stream is ordered after
-    // every part's last chunk through the hand-off events
-    if (np > 1 && hipMemcpyAsync(c->x, head->x, sizeof(float) * (size_t)T * E, hipMemcpyDeviceToDevice, hs) != hipSuccess) {
+    // every stage's last piece through the hand-off events
+    if (xl != c->x && hipMemcpyAsync(c->x, xl, sizeof(float) * (size_t)T * E, hipMemcpyDeviceToDevice, hs) != hipSuccess) {
         snprintf(err, errlen, "hidden copy failed"); return fail_sync();
     }
-    if (!wait) {   // a single part: the head stream is the chain's
+    if (!wait) {   // one chunk; the head's stream
         const int nl = nlog < T ? nlog : T;
         if (hipMemcpyAsync(c->h_buf, c->d_argmax, 4 * nl, hipMemcpyDeviceToHost, hs) != hipSuccess) {
             snprintf(err, errlen, "argmax copy failed"); return fail_sync();

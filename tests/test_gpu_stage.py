@@ -427,3 +427,56 @@ def test_prefill_chunk_with_checkpoints_rolls_back(tiny):
     for s_ in (g, ref, c):
         s_.destroy()
 
+
+
+@pytest.mark.parametrize("T", [65, 96, 129, 200, 256])
+def test_wide_chunk_equals_chunks_of_64(tiny, T):
+    """A chunk beyond 64 tokens takes the wide GEMM (256 x 128 tiles over
+    every segment, token tiles of 32: 65 = two and a row, 129 = a second
+    token group of one token) and attention in slices; its hidden rows are
+    those of the same tokens in chunks of 64 on the other GEMM, and the state
+    it leaves serves a decode step. Both round only in fp32 sums: 1e-6 of a
+    product, 6e-6 after four layers."""
+    m, L = tiny, tiny.hp.n_layer
+    toks = prompt_ids(m, T + 1, 300 + T)
+    a = xp.HipStage(m, 0, L, 320, 256, True)
+    b = xp.HipStage(m, 0, L, 320, 64, True)
+    x = embed(m, toks[:T])
+    ya = a.forward(x.copy())
+    yb = np.concatenate([b.forward(x[i:i + 64].copy()) for i in range(0, T, 64)])
+    assert rel_l2(ya, yb) < 5e-5
+    x1 = embed(m, toks[T:])
+    assert rel_l2(a.forward(x1.copy()), b.forward(x1.copy())) < 5e-5
+    c = orc.CpuStage(m.ptr, 0, L, 320, 256, True, kv_f16=True)
+    assert rel_l2(ya, c.forward(x.copy())) < 1e-3
+    for s in (a, b, c):
+        s.destroy()
+
+
+@pytest.mark.parametrize("n,mb", [(40, 16), (200, 16), (31, 8), (33, 8), (1030, 64), (1601, 64)])
+def test_chain_prompt_pieces(tiny, n, mb):
+    """A prompt beyond max_batch goes through the layers in pieces of up to
+    1024 tokens (1030: 512 + 518, so that the last piece holds max_batch
+    rows; below 32 tokens with max_batch 8 on the GEMV): the logits of its
+    last rows are those of the vtable's chunks, one chain of two stages gives
+    them bit for bit, and decoding continues from its state."""
+    m, L = tiny, tiny.hp.n_layer
+    prompt = prompt_ids(m, n, 400 + n)
+    one = xp.HipStage(m, 0, L, 2048, mb, True)
+    c1 = xp.Chain([one])
+    nl = min(3, n - (n - 1) // mb * mb)
+    am1, lg1 = c1.eval(prompt, nlog=3, want_logits=True)
+    ref = xp.HipStage(m, 0, L, 2048, mb, True)
+    x = embed(m, prompt)
+    y = np.concatenate([ref.forward(x[i:i + mb].copy()) for i in range(0, n, mb)])
+    want = ref.logits(y[-nl:])
+    assert rel_l2(lg1[:nl], want) < 2e-4
+    sts = [xp.HipStage(m, 0, 3, 2048, mb, False), xp.HipStage(m, 3, L, 2048, mb, True)]
+    c2 = xp.Chain(sts)
+    am2, lg2 = c2.eval(prompt, nlog=3, want_logits=True)
+    assert np.array_equal(lg1[:nl].view(np.uint32), lg2[:nl].view(np.uint32))
+    assert c2.decode(6).tolist() == c1.decode(6).tolist()
+    for c in (c1, c2):
+        c.free()
+    for s in [one, ref] + sts:
+        s.destroy()
