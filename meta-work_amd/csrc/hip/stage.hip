@@ -122,11 +122,31 @@ int env_int(const char *k, int def) {
 
 HStage *H(xj_stage *s) { return reinterpret_cast<HStage *>(s); }
 
+// The kept work area of xjh_delta_chunked, of at most kKeepWork bytes; given
+// back when the library finds no memory for something else (device_alloc).
+constexpr size_t kKeepWork = size_t(512) << 20;
+struct KeptWork {
+    std::mutex mu;
+    void *p = nullptr;
+    size_t cap = 0;
+} g_work;
+
+bool device_alloc(void **p, size_t bytes) {
+    if (hipMalloc(p, bytes) == hipSuccess) return true;
+    std::unique_lock<std::mutex> lock(g_work.mu, std::try_to_lock);
+    if (!lock.owns_lock() || !g_work.p) return false;
+    (void)hipFree(g_work.p);
+    g_work.p = nullptr;
+    g_work.cap = 0;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes) == hipSuccess;
+}
+
 template <class T>
 T *dalloc(HStage *S, size_t n, char *err, size_t errlen) {
     void *p = nullptr;
     if (n == 0) n = 1;
-    if (hipMalloc(&p, n * sizeof(T)) != hipSuccess) {
+    if (!device_alloc(&p, n * sizeof(T))) {
         snprintf(err, errlen, "HBM allocation of %zu bytes failed", n * sizeof(T));
         return nullptr;
     }
@@ -2235,7 +2255,7 @@ int ops_done(char *err, size_t errlen) {
 
 extern "C" void *xjh_malloc(size_t bytes) {
     void *p = nullptr;
-    if (hipMalloc(&p, bytes ? bytes : 1) != hipSuccess) { snprintf(g_lasterr, sizeof g_lasterr, "hipMalloc(%zu) failed", bytes); return nullptr; }
+    if (!device_alloc(&p, bytes ? bytes : 1)) { snprintf(g_lasterr, sizeof g_lasterr, "hipMalloc(%zu) failed", bytes); return nullptr; }
     return p;
 }
 extern "C" void xjh_free(void *p) { if (p) (void)hipFree(p); }
@@ -2250,7 +2270,7 @@ extern "C" void *xjh_upload_weight(uint32_t type, const void *host, int64_t n_ro
     if (!gemv_type_ok(type)) { snprintf(err, errlen, "type %s has no device layout", xjh_type_name(type)); return nullptr; }
     const uint64_t bytes = xjh_row_bytes(type, k) * (uint64_t)n_rows;
     void *p = nullptr;
-    if (hipMalloc(&p, bytes + kWeightPad) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return nullptr; }
+    if (!device_alloc(&p, bytes + kWeightPad)) { snprintf(err, errlen, "hipMalloc failed"); return nullptr; }
     if (upload_repack(type, host, n_rows, k, (uint8_t *)p, g_stream, err, errlen)) { (void)hipFree(p); return nullptr; }
     return p;
 }
@@ -2626,11 +2646,26 @@ extern "C" int xjh_delta_chunked(int H, int S, int T, int chunk, const float *q,
     if (!ops_stream()) return -1;
     const size_t wb = delta_chunked_work_bytes(H, S, T, chunk);
     if (!wb) { snprintf(err, errlen, "chunked delta: unsupported shape (S=%d, chunk=%d)", S, chunk); return -1; }
-    void *work = nullptr;
-    if (hipMalloc(&work, wb) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+    // the work area: kept between calls up to kKeepWork bytes (allocating and freeing 75 MB costs 400 us, twice
+    // the kernels of a 2048-token call), one at a time; a call beside another, or a larger one, has its own
+    std::unique_lock<std::mutex> lock(g_work.mu, std::try_to_lock);
+    void *own = nullptr, *work = nullptr;
+    if (lock.owns_lock() && wb <= kKeepWork) {
+        if (wb > g_work.cap) {
+            if (g_work.p) (void)hipFree(g_work.p);
+            g_work.p = nullptr;
+            g_work.cap = 0;
+            if (hipMalloc(&g_work.p, wb) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+            g_work.cap = wb;
+        }
+        work = g_work.p;
+    } else {
+        if (hipMalloc(&own, wb) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+        work = own;
+    }
     int rc = delta_chunked_launch(H, S, T, chunk, q, k, v, decay, beta, qscale, state, out, (float *)work, g_stream);
     if (rc) snprintf(err, errlen, "chunked delta launch failed (q, k, v and state must be 16-byte aligned)");
     else rc = ops_done(err, errlen);
-    (void)hipFree(work);
+    if (own) (void)hipFree(own);
     return rc;
 }

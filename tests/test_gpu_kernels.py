@@ -242,3 +242,25 @@ def test_delta_prefill_then_decode():
     assert rel_l2(go0, oo[:T0]) < 1e-3
     assert rel_l2(np.concatenate(outs), oo[T0:]) < 1e-3
     assert rel_l2(gst, ost) < 1e-3
+
+
+@pytest.mark.parametrize("S", [64, 128])
+@pytest.mark.parametrize("T", [1, 16, 17, 63, 64, 65, 127, 129])
+def test_delta_chunked_edges(S, T):
+    """Chunk edges of the chunked rule (one token, the 16-token blocks of its
+    inverse, a chunk less one, one and two chunks and a token) from a
+    non-zero state, both state sizes: fp32 sums of at most 64 + 128 terms per
+    chunk, 8e-7 of float64 measured over three chunks."""
+    H = 5
+    q, k, v, dec, beta = _delta_inputs(T, H, S, 7 * T + S)
+    st0 = np.random.default_rng(T).standard_normal((H, S, S)).astype(np.float32) * 0.1
+    qs = 1 / np.sqrt(S)
+    go, gs = xp.delta(q, k, v, dec, beta, st0, qs, chunk=64)
+    m, oo = st0.astype(np.float64), np.empty((T, H, S))
+    for t in range(T):
+        m *= dec[t].astype(np.float64)[:, None, None]
+        d = (v[t] - np.einsum("hji,hi->hj", m, k[t])) * beta[t][:, None]
+        m += d[:, :, None] * k[t][:, None, :]
+        oo[t] = np.einsum("hji,hi->hj", m, q[t]) * qs
+    assert rel_l2(go, oo) < 5e-6
+    assert rel_l2(gs, m) < 5e-6
