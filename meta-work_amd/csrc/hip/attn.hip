@@ -443,6 +443,249 @@ static int launch_d(const AttnArgs &a, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+// ------------------------------------------------- chunks of a prompt --
+// Causal attention of T tokens over the prefix on the matrix cores (chunks of
+// 16 tokens and more; the split kernel above computes every score on the
+// vector units and reads a kv head's keys once per token: 16 heads of 256,
+// 1024 tokens: 440 us of it and 193 us of its combine per layer, against 70 us).
+// The longest work-group's tiles bound it, each a chain of loads, scores,
+// softmax and products at one wavefront per SIMD (4 us).
+// A work-group takes 64 query rows of one kv head (64 / G tokens x G heads)
+// and walks a split of the positions in tiles of 64, a wavefront 16 rows.
+// Scores come transposed, S^T = K Q^T (v_mfma_f32_16x16x32_f16: keys as rows of
+// the tile, query rows as columns), so a lane holds one query row's scores and
+// the softmax state is per lane; its 8 scores of a 32-key step are, with the
+// step's keys taken in the order 4 kq + r, 16 + 4 kq + r, the operand of
+// O^T = V^T P^T as they are. Keys and values are the cache's fp16, exact
+// operands; queries and probabilities, fp32, enter as two f16 planes each
+// (about 22 bits: x 2^-e = hi + lo, e per query row; p 2^14 = hi + lo), the
+// sums are fp32. K tiles lie row by row in LDS, V tiles transposed (8 x 8
+// blocks turned in registers), both with their 16-byte pieces permuted so that
+// 16 lanes read distinct banks; the next tile is in flight meanwhile.
+typedef _Float16 hf8 __attribute__((ext_vector_type(8)));
+typedef float f32x4_ __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4_ mfma16(hf8 a, hf8 b, f32x4_ c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ void split2(float x, _Float16 &hi, _Float16 &lo) {
+    hi = (_Float16)x;
+    lo = (_Float16)(x - (float)hi);   // x - hi is exact in fp32
+}
+
+template <int D, int G>
+__global__ __launch_bounds__(256, 1) void attn_chunk_kernel(const AttnArgs a) {
+    constexpr int CH = D / 8;                 // 16-byte pieces per key
+    constexpr int KP = CH / 4;                // K pieces per thread and tile
+    constexpr int RS = CH >= 16 ? 0 : 1;      // rows sharing 256 bytes (log2)
+    constexpr int TQ = 64 / G;                // tokens per work-group
+    constexpr int NS = D / 32, ND = D / 16;   // inner steps of a score, 16-dim tiles of the output
+    __shared__ __align__(16) uint8_t Ks[64 * D * 2];
+    __shared__ __align__(16) uint8_t Vt[D * 128];
+    const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, li = l & 15, kq = l >> 4;
+    const int g = blockIdx.y, sp = blockIdx.z, nk = a.Hkv * D;
+    const int tb = ((int)gridDim.x - 1 - (int)blockIdx.x) * TQ;   // the longest rows first
+    const int npast = *a.npast + a.t0;
+    const int last = npast + min(tb + TQ, a.T) - 1;               // the work-group's last position
+    const int k0 = sp * a.sp, k1 = min(k0 + a.sp, last + 1);
+    if (k0 > last) return;
+    const int row = 16 * w + li, t = tb + row / G, h = g * G + row % G, tc = min(t, a.T - 1);
+    const int pos = npast + tc;
+    // this lane's query row: dims 32 s + 8 kq .. + 7 in two planes
+    hf8 qh[NS], ql[NS];
+    float qsc;
+    {
+        const float *qp = a.qr + ((int64_t)tc * a.H + h) * D + 8 * kq;
+        float m = 0.f;
+        f32x4_ v[NS][2];
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                v[s][i] = *(const f32x4_ *)(qp + 32 * s + 4 * i);
+#pragma unroll
+                for (int c = 0; c < 4; c++) m = fmaxf(m, fabsf(v[s][i][c]));
+            }
+        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        int E = 0;
+        (void)frexpf(m, &E);   // m < 2^E
+        if (E < -100) E = -100;
+        const int e = E - 14;
+#pragma unroll
+        for (int s = 0; s < NS; s++)
+#pragma unroll
+            for (int c = 0; c < 8; c++) {
+                _Float16 hi, lo;
+                split2(ldexpf(v[s][c >> 2][c & 3], -e), hi, lo);
+                qh[s][c] = hi;
+                ql[s][c] = lo;
+            }
+        qsc = ldexpf(1.f, e);
+    }
+    u32x4 kr[KP], vr[8];
+    const int kc = tid % CH, kr0 = tid / CH;
+    const bool vt = tid < 8 * CH;             // D < 256: the first 8 CH threads turn the values
+    const int vdb = tid % CH, vkb = (tid / CH) & 7;
+    auto load = [&](int j0) {   // the tile's keys and values, clamped to written positions
+#pragma unroll
+        for (int p = 0; p < KP; p++) {
+            const int r = min(j0 + kr0 + (256 / CH) * p, last);
+            kr[p] = *(const u32x4 *)(a.kc + (int64_t)r * nk + g * D + 8 * kc);
+        }
+        if (vt)
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const int r = min(j0 + 32 * (vkb >> 2) + 16 * (i >> 2) + 4 * (vkb & 3) + (i & 3), last);
+                vr[i] = *(const u32x4 *)(a.vc + (int64_t)r * nk + g * D + 8 * vdb);
+            }
+    };
+    auto kaddr = [&](int r, int c) { return r * (D * 2) + 16 * (c ^ ((r >> RS) & (CH < 16 ? CH - 1 : 15))); };
+    auto vaddr = [&](int d, int c) { return d * 128 + 16 * (c ^ (((d >> 1) ^ (d >> 4)) & 7)); };
+    f32x4_ o[ND];
+#pragma unroll
+    for (int d = 0; d < ND; d++) o[d] = f32x4_{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, lsum = 0.f;
+    load(k0);
+    for (int j0 = k0; j0 < k1; j0 += 64) {
+        __syncthreads();   // the previous tile is used
+#pragma unroll
+        for (int p = 0; p < KP; p++) *(u32x4 *)(Ks + kaddr(kr0 + (256 / CH) * p, kc)) = kr[p];
+        if (vt)
+#pragma unroll
+            for (int c = 0; c < 4; c++) {   // dims 8 vdb + 2 c and + 1 of the thread's 8 keys
+                u32x4 x, y;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    x[i] = __builtin_amdgcn_perm(vr[2 * i + 1][c], vr[2 * i][c], 0x05040100u);
+                    y[i] = __builtin_amdgcn_perm(vr[2 * i + 1][c], vr[2 * i][c], 0x07060302u);
+                }
+                *(u32x4 *)(Vt + vaddr(8 * vdb + 2 * c, vkb)) = x;
+                *(u32x4 *)(Vt + vaddr(8 * vdb + 2 * c + 1, vkb)) = y;
+            }
+        __syncthreads();
+        if (j0 + 64 < k1) load(j0 + 64);
+        f32x4_ s[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) s[u] = f32x4_{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int st = 0; st < NS; st++) {
+            hf8 ka[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) ka[u] = *(const hf8 *)(Ks + kaddr(16 * u + li, 4 * st + kq));
+#pragma unroll
+            for (int u = 0; u < 4; u++) s[u] = mfma16(ka[u], ql[st], s[u]);
+#pragma unroll
+            for (int u = 0; u < 4; u++) s[u] = mfma16(ka[u], qh[st], s[u]);
+        }
+        // register r of s[u]: key j0 + 16 u + 4 kq + r of this lane's query row
+        float mt = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float x = s[u][r] * qsc * a.scale;
+                s[u][r] = j0 + 16 * u + 4 * kq + r <= pos ? x : -INFINITY;
+                mt = fmaxf(mt, s[u][r]);
+            }
+        mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+        const float mn = fmaxf(m, mt), ms = mn == -INFINITY ? 0.f : mn;   // (a row with no key yet: all terms 0)
+        const float al = expf(m - ms);
+        m = mn;
+        float lt = 0.f;
+        hf8 ph[2], pl[2];
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float p = expf(s[u][r] - ms);
+                lt += p;
+                _Float16 hi, lo;
+                split2(p * 16384.f, hi, lo);
+                ph[u >> 1][4 * (u & 1) + r] = hi;
+                pl[u >> 1][4 * (u & 1) + r] = lo;
+            }
+        lt += __shfl_xor(lt, 16, 64);
+        lt += __shfl_xor(lt, 32, 64);
+        lsum = lsum * al + lt;
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            o[d] *= al;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const hf8 va = *(const hf8 *)(Vt + vaddr(16 * d + li, 4 * j + kq));
+                o[d] = mfma16(va, pl[j], o[d]);
+                o[d] = mfma16(va, ph[j], o[d]);
+            }
+        }
+    }
+    if (t >= a.T) return;
+    constexpr float kP = 1.f / 16384.f;
+    if (a.n_chunk_sp > 1) {   // register r of o[d]: dim 16 d + 4 kq + r
+        float *part = a.scores + (((int64_t)t * a.H + h) * a.n_chunk_sp + sp) * (D + 4);
+#pragma unroll
+        for (int d = 0; d < ND; d++) *(f32x4_ *)(part + 4 + 16 * d + 4 * kq) = o[d] * kP;
+        if (kq == 0) part[0] = m, part[1] = lsum;
+    } else {
+        const float inv = 1.0f / lsum;
+        const float *gp = a.qg + (int64_t)t * a.qg_s + (int64_t)h * 2 * D + D + 4 * kq;
+        float *op = a.out + (int64_t)t * a.H * D + (int64_t)h * D + 4 * kq;
+#pragma unroll
+        for (int d = 0; d < ND; d++) {
+            f32x4_ v;
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = o[d][r] * kP * inv * xjd::sigm(gp[16 * d + r]);
+            *(f32x4_ *)(op + 16 * d) = v;
+        }
+    }
+}
+
+// The splits of attn_chunk_kernel merged, as attn_combine_kernel merges its own.
+template <int D>
+__global__ __launch_bounds__(D) void attn_chunk_merge_kernel(const AttnArgs a) {
+    const int h = blockIdx.x, t = blockIdx.y, d = threadIdx.x;
+    const float *part = a.scores + ((int64_t)t * a.H + h) * a.n_chunk_sp * (D + 4);
+    const float gx = a.qg[(int64_t)t * a.qg_s + (int64_t)h * 2 * D + D + d];
+    const int ns = (*a.npast + a.t0 + t) / a.sp + 1;
+    float M = -INFINITY;
+    for (int s = 0; s < ns; s++) M = fmaxf(M, part[s * (D + 4)]);
+    float o = 0.f, L = 0.f;
+    for (int s = 0; s < ns; s++) {
+        const float f = expf(part[s * (D + 4)] - M);
+        L = fmaf(f, part[s * (D + 4) + 1], L);
+        o = fmaf(f, part[s * (D + 4) + 4 + d], o);
+    }
+    a.out[(int64_t)t * a.H * D + (int64_t)h * D + d] = o * (1.0f / L) * xjd::sigm(gx);
+}
+
+template <int D, int G>
+static void launch_chunk_g(const AttnArgs &in, int n_past, int64_t score_floats, hipStream_t st) {
+    AttnArgs a = in;
+    const int nt = (a.T + 64 / G - 1) / (64 / G), keys = n_past + a.T, tiles = (keys + 63) / 64;
+    // splits of the positions until about two work-groups per CU exist, within the scratch
+    // splits of the positions until there is a work-group per CU, within the scratch (1024 tokens of 4 kv heads:
+    // unsplit 70 us, in two 71 us and 22 us of merging; 64 tokens at 960: 16 splits, 14.5 + 9 us, against 42 + 16)
+    int ns = 256 / (nt * a.Hkv);
+    const int64_t cap = score_floats / ((int64_t)a.T * a.H * (D + 4));
+    if (ns > cap) ns = (int)cap;
+    if (ns > tiles) ns = tiles;
+    if (ns < 1) ns = 1;
+    a.sp = (tiles + ns - 1) / ns * 64;
+    a.n_chunk_sp = (keys + a.sp - 1) / a.sp;
+    hipLaunchKernelGGL((attn_chunk_kernel<D, G>), dim3(nt, a.Hkv, a.n_chunk_sp), dim3(256), 0, st, a);
+    if (a.n_chunk_sp > 1) hipLaunchKernelGGL(attn_chunk_merge_kernel<D>, dim3(a.H, a.T), dim3(D), 0, st, a);
+}
+template <int D>
+static int launch_chunk(const AttnArgs &a, int n_past, int64_t score_floats, hipStream_t st) {
+    hipLaunchKernelGGL(kv_store_kernel<D>, dim3(a.T, a.Hkv), dim3(256), 0, st, a);
+    switch (a.H / a.Hkv) {
+    case 1: launch_chunk_g<D, 1>(a, n_past, score_floats, st); break;
+    case 2: launch_chunk_g<D, 2>(a, n_past, score_floats, st); break;
+    case 4: launch_chunk_g<D, 4>(a, n_past, score_floats, st); break;
+    default: launch_chunk_g<D, 8>(a, n_past, score_floats, st); break;
+    }
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 // NeoX RoPE in place (xj_cpu.c:68-77) of T tokens x n_heads heads, one
 // thread per pair (i, i + n_rot/2), with cos and sin of position pos0 + t from
 // the same kind of table kv_store reads (cs[t][n_rot/2]).
@@ -480,12 +723,28 @@ int rope_launch(float *x, const float2 *cs, int T, int n_heads, int64_t tok_stri
 
 int attn_splits(int n_ctx) { return (n_ctx + kSplitP - 1) / kSplitP; }
 
-int attn_launch(const AttnArgs &a, hipStream_t st) {
+static bool attn_args_ok(const AttnArgs &a) {
     const int G = a.Hkv > 0 ? a.H / a.Hkv : 0;
-    if (a.Hkv < 1 || a.H % a.Hkv || (G != 1 && G != 2 && G != 4 && G != 8) || a.n_rot > a.D || a.n_rot % 2 ||
-        a.n_split != attn_splits(a.n_ctx) ||
-        !a.qr)
+    return a.Hkv >= 1 && a.H % a.Hkv == 0 && (G == 1 || G == 2 || G == 4 || G == 8) && a.n_rot <= a.D && a.n_rot % 2 == 0 &&
+           a.n_split == attn_splits(a.n_ctx) && a.qr;
+}
+
+// T tokens at positions n_past .. (n_past = *a.npast + a.t0, known to the
+// caller) on the matrix cores; scores holds score_floats floats; xq is not written.
+int attn_chunk_launch(const AttnArgs &a, int n_past, int64_t score_floats, hipStream_t st) {
+    if (!attn_args_ok(a) || a.T < 1 || n_past < 0 || n_past + a.T > a.n_ctx || !a.scores ||
+        (((uintptr_t)a.kc | (uintptr_t)a.vc | (uintptr_t)a.qr | (uintptr_t)a.scores | (uintptr_t)a.out) & 15))
         return -1;
+    switch (a.D) {
+    case 64: return launch_chunk<64>(a, n_past, score_floats, st);
+    case 128: return launch_chunk<128>(a, n_past, score_floats, st);
+    case 256: return launch_chunk<256>(a, n_past, score_floats, st);
+    default: return -1;
+    }
+}
+
+int attn_launch(const AttnArgs &a, hipStream_t st) {
+    if (!attn_args_ok(a)) return -1;
     switch (a.D) {
     case 64: return launch_d<64>(a, st);
     case 128: return launch_d<128>(a, st);

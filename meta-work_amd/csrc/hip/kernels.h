@@ -226,8 +226,10 @@ struct AttnArgs {
     float eps, scale;
     uint8_t *xq;                         // optional: prepared activations of out (no prologue)
     int32_t t0;                          // token 0 sits at position *npast + t0
+    int32_t sp, n_chunk_sp;              // set by attn_chunk_launch: positions per split, splits
 };
 int attn_launch(const AttnArgs &a, hipStream_t st);
+int attn_chunk_launch(const AttnArgs &a, int n_past, int64_t score_floats, hipStream_t st);
 int attn_splits(int n_ctx);             // 64-position splits covering n_ctx
 
 struct DeltaArgs {

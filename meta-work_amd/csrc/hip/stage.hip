@@ -95,6 +95,7 @@ struct HStage {
     // prefill on the matrix cores: per-token RMSNorm scales, the GEMM's K-split
     // partials and the chunked delta rule's work area
     float *tsc = nullptr, *gpart = nullptr, *dwork = nullptr;
+    int64_t score_floats = 0;
     uint8_t *hq = nullptr;     // the GEMM's activations, max_batch tokens of the largest input
     int64_t gpart_floats = 0;
     int32_t *gcnt = nullptr;   // the GEMM's arrival counters (zero between launches)
@@ -567,19 +568,23 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
         at.n_split = attn_splits(S->s.n_ctx);
         at.eps = hp.eps; at.scale = 1.0f / sqrtf((float)D);
         Gemv q = gemv(S->xq_att);
-        q.a.x = S->o; q.a.xs = Hq * D; q.a.pro = PRO_NONE;
         q.seg(L.wo, x, E, EPI_ADD);
-        q.prepared = !q.wide_ok(T);
-        if (q.prepared) q.a.x = nullptr;
-        // long pieces in slices of 64 tokens (the split partials' scratch)
-        for (int t0 = 0; !pf && t0 < T; t0 += kAttnT) {
-            AttnArgs b = at;
-            b.t0 = t0;
-            b.T = T - t0 < kAttnT ? T - t0 : kAttnT;
-            b.qg += (int64_t)t0 * at.qg_s; b.kn += (int64_t)t0 * at.kn_s; b.vn += (int64_t)t0 * at.vn_s;
-            b.out += (int64_t)t0 * Hq * D;
-            b.xq = q.prepared ? S->xq_att + (int64_t)t0 * xq_off(Hq * D).stride : nullptr;
-            if (attn_launch(b, st)) return -1;
+        // chunks on the matrix cores leave wo's input to its own prep launch; shorter ones, and those kept on
+        // the GEMV's arithmetic, take the decode kernels, in slices of the split partials' scratch
+        if (!pf && T >= S->gemm_min) {
+            if (attn_chunk_launch(at, S->s.n_past, S->score_floats, st)) return -1;
+            q.a.x = S->o; q.a.xs = Hq * D; q.a.pro = PRO_NONE;
+        } else {
+            q.prepared = true;
+            for (int t0 = 0; !pf && t0 < T; t0 += kAttnT) {
+                AttnArgs b = at;
+                b.t0 = t0;
+                b.T = T - t0 < kAttnT ? T - t0 : kAttnT;
+                b.qg += (int64_t)t0 * at.qg_s; b.kn += (int64_t)t0 * at.kn_s; b.vn += (int64_t)t0 * at.vn_s;
+                b.out += (int64_t)t0 * Hq * D;
+                b.xq = S->xq_att + (int64_t)t0 * xq_off(Hq * D).stride;
+                if (attn_launch(b, st)) return -1;
+            }
         }
         if (q.run(T, st)) return -1;
     }
@@ -836,7 +841,8 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
     S->g = dalloc<float>(S, mb * sf, err, errlen);
     S->u = dalloc<float>(S, mb * sf, err, errlen);
     S->qr = dalloc<float>(S, mb * hp.n_head * (size_t)hp.head_dim, err, errlen);
-    S->scores = dalloc<float>(S, (mb < kAttnT ? mb : kAttnT) * hp.n_head * (size_t)attn_splits(n_ctx) * (hp.head_dim + 2), err, errlen);
+    S->score_floats = (int64_t)(mb < kAttnT ? mb : kAttnT) * hp.n_head * attn_splits(n_ctx) * (hp.head_dim + 2);
+    S->scores = dalloc<float>(S, (size_t)S->score_floats, err, errlen);
     S->npast = dalloc<int32_t>(S, 1, err, errlen);
     // prefill on the matrix cores (chunks of at least 16 tokens)
     S->tsc = dalloc<float>(S, mb, err, errlen);
@@ -1412,6 +1418,7 @@ static int chain_eval(xjh_chain *c, const int32_t *tokens, int n, int nlog, int 
                 R = c->twins[i];
                 R->L = S->L;   // checkpoint and snapshot buffers allocated since
                 R->gemm_min = gemm_min;
+                R->s.n_past = S->s.n_past;
                 S->s.keep = 0;
                 S->s.ck_start = S->s.n_past;
                 S->s.ck_T = 0;
