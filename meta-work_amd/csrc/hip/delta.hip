@@ -220,6 +220,112 @@ __global__ __launch_bounds__(S) void delta_prefill_prep_kernel(const DeltaPrepAr
     }
 }
 
+// The same from the raw qkv projections of a prompt chunk: the depthwise causal
+// conv + SiLU of the three parts (conv_silu_kernel's expressions; inputs before
+// the chunk from the conv state, which stays as it is) and the L2 norms in one
+// pass. A wavefront takes one value head and kConvT tokens, a lane S / 64
+// channels of q, k and v each, every input requested at once; q and k are
+// formed again for each value head of a key head. (Walking the tokens per
+// channel, 192 wavefronts of a 12288-channel layer: 126 us for 1024 tokens and
+// 33 us for the norms; in one pass 33 us.)
+constexpr int kConvT = 8;
+
+template <int S, int KC>
+__global__ __launch_bounds__(64) void delta_conv_prep_kernel(const DeltaPrepArgs a) {
+    constexpr int NE = S / 64;
+    const int t0 = blockIdx.x * kConvT, hv = blockIdx.y, l = threadIdx.x, hk = hv % a.Hk;
+    const int ch[3] = {hk * S + NE * l, a.k_off + hk * S + NE * l, a.v_off + hv * S + NE * l};
+    float x[3][KC - 1 + kConvT][NE], w[3][NE][KC];
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+#pragma unroll
+        for (int i = 0; i < KC - 1 + kConvT; i++) {
+            const int t = t0 + i - (KC - 1);
+            const float *src = a.qkv + (int64_t)min(max(t, 0), a.T - 1) * a.qkv_s + ch[p];
+#pragma unroll
+            for (int e = 0; e < NE; e++) x[p][i][e] = src[e];
+        }
+#pragma unroll
+        for (int e = 0; e < NE; e++)
+#pragma unroll
+            for (int k = 0; k < KC; k++) w[p][e][k] = a.conv_w[(int64_t)(ch[p] + e) * KC + k];
+    }
+    if (t0 < KC - 1) {   // (uniform) inputs before the chunk: the state holds the last KC - 1
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+#pragma unroll
+            for (int i = 0; i < KC - 1; i++)
+                if (t0 + i < KC - 1)
+#pragma unroll
+                    for (int e = 0; e < NE; e++) x[p][i][e] = a.conv_state[(int64_t)(ch[p] + e) * (KC - 1) + t0 + i];
+    }
+#pragma unroll
+    for (int j = 0; j < kConvT; j++) {
+        const int t = t0 + j;
+        if (t >= a.T) break;   // uniform
+        float y[3][NE];
+#pragma unroll
+        for (int p = 0; p < 3; p++)
+#pragma unroll
+            for (int e = 0; e < NE; e++) {
+                float s = 0.f;
+#pragma unroll
+                for (int k = 0; k < KC; k++) s = fmaf(x[p][j + k][e], w[p][e][k], s);
+                y[p][e] = xjd::silu(s);
+            }
+        double sq = 0, sk = 0;
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            sq += (double)y[0][e] * y[0][e];
+            sk += (double)y[1][e] * y[1][e];
+        }
+        const float qn = 1.0f / sqrtf((float)xjd::wave_sum_d(sq) + a.eps), kn = 1.0f / sqrtf((float)xjd::wave_sum_d(sk) + a.eps);
+        const int64_t o = ((int64_t)t * a.Hv + hv) * S + NE * l;
+#pragma unroll
+        for (int e = 0; e < NE; e++) {
+            a.q[o + e] = y[0][e] * qn;
+            a.k[o + e] = y[1][e] * kn;
+            a.v[o + e] = y[2][e];
+        }
+    }
+    if (l < kConvT && t0 + l < a.T) {
+        const int64_t t = t0 + l;
+        a.decay[t * a.Hv + hv] = expf(xjd::softplus(a.alpha[t * a.alpha_s + hv] + a.dt[hv]) * a.A[hv]);
+        a.bt[t * a.Hv + hv] = xjd::sigm(a.beta[t * a.beta_s + hv]);
+    }
+}
+
+// The conv state after the chunk: its last KC - 1 inputs (T >= KC - 1).
+__global__ __launch_bounds__(256) void conv_tail_kernel(const float *x, int64_t xs, int T, int C, int n, float *state) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;   // state element [channel][n]
+    if (i >= (int64_t)C * n) return;
+    state[i] = x[(int64_t)(T - n + i % n) * xs + i / n];
+}
+
+template <int S>
+static void conv_prep_launch(const DeltaPrepArgs &a, int KC, hipStream_t st) {
+    const dim3 g((a.T + kConvT - 1) / kConvT, a.Hv), b(64);
+    switch (KC) {
+    case 2: hipLaunchKernelGGL((delta_conv_prep_kernel<S, 2>), g, b, 0, st, a); break;
+    case 3: hipLaunchKernelGGL((delta_conv_prep_kernel<S, 3>), g, b, 0, st, a); break;
+    case 4: hipLaunchKernelGGL((delta_conv_prep_kernel<S, 4>), g, b, 0, st, a); break;
+    case 5: hipLaunchKernelGGL((delta_conv_prep_kernel<S, 5>), g, b, 0, st, a); break;
+    case 6: hipLaunchKernelGGL((delta_conv_prep_kernel<S, 6>), g, b, 0, st, a); break;
+    case 7: hipLaunchKernelGGL((delta_conv_prep_kernel<S, 7>), g, b, 0, st, a); break;
+    default: hipLaunchKernelGGL((delta_conv_prep_kernel<S, 8>), g, b, 0, st, a); break;
+    }
+}
+int delta_conv_prep_launch(const DeltaPrepArgs &a, int C, int KC, hipStream_t st) {
+    if (a.T < 8 || a.Hk < 1 || a.Hv < 1 || KC < 2 || KC > 8 || C < 1 || !a.conv_state || !a.conv_w) return -1;
+    if (a.S == 128) conv_prep_launch<128>(a, KC, st);
+    else if (a.S == 64) conv_prep_launch<64>(a, KC, st);
+    else return -1;
+    const int n = KC - 1;
+    hipLaunchKernelGGL(conv_tail_kernel, dim3((unsigned)(((int64_t)C * n + 255) / 256)), dim3(256), 0, st, a.qkv, (int64_t)a.qkv_s,
+                       a.T, C, n, a.conv_state);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 int delta_prefill_prep_launch(const DeltaPrepArgs &a, hipStream_t st) {
     if (a.T < 1 || a.Hk < 1 || a.Hv < 1) return -1;
     if (a.S == 128) hipLaunchKernelGGL(delta_prefill_prep_kernel<128>, dim3(a.T, a.Hv), dim3(128), 0, st, a);

@@ -265,8 +265,13 @@ struct DeltaPrepArgs {
     float *q, *k, *v, *decay, *bt;
     int32_t T, Hk, Hv, S;
     float eps;
+    float *conv_state;            // delta_conv_prep_launch: [C][KC-1]
+    const float *conv_w;          // [C][KC]
 };
 int delta_prefill_prep_launch(const DeltaPrepArgs &a, hipStream_t st);
+// The same from projections qkv before the conv + SiLU (kernel KC <= 8, C
+// channels, T >= 8), whose state advances by the T tokens.
+int delta_conv_prep_launch(const DeltaPrepArgs &a, int C, int KC, hipStream_t st);
 
 // Standalone gated delta rule (decay/beta given), recurrent and chunked.
 int delta_recurrent_launch(int H, int S, int T, const float *q, const float *k, const float *v,
@@ -282,7 +287,7 @@ size_t delta_chunked_work_bytes(int H, int S, int T, int chunk);
 // rollbacks to a checkpoint). Entries past kCopyMax take further launches.
 constexpr int kCopyMax = 48;
 struct CopyList {
-    const float *src[kCopyMax];
+    const float *src[kCopyMax];   // null: dst is set to zero
     float *dst[kCopyMax];
     int64_t n[kCopyMax];   // floats
     int32_t cnt;

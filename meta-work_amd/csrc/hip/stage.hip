@@ -282,6 +282,7 @@ struct Gemv {
     uint8_t *hq = nullptr;
     bool hq_ready = false;
     bool hq_out = false;   // set by a GEMM run whose SwiGLU prep built the next input's hq
+    bool raw_conv = false; // a GEMM run leaves the conv segment's projections as they are
     const WideBuf *wide = nullptr;
     int gemm_min = kGemmMinT;
     // Chunks of at least kGemmMinT tokens take the matrix-core GEMM
@@ -416,7 +417,7 @@ struct Gemv {
                 }
             }
             // depthwise causal conv + SiLU over the T tokens, with its state and checkpoints
-            if (s.epi == EPI_CONV &&
+            if (s.epi == EPI_CONV && !raw_conv &&
                 conv_silu_launch(s.y, s.conv_state, s.conv_w, s.n_rows, s.conv_k, T, s.conv_ck, a.keep_n, st))
                 return -1;
         }
@@ -502,21 +503,25 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
          .seg(L.ssm_beta, S->beta, Hv, EPI_STORE).seg(L.ssm_alpha, S->alpha, Hv, EPI_STORE);
         GSeg &cs = p.a.seg[0];
         cs.conv_state = L.conv; cs.conv_w = L.conv_w; cs.conv_ck = L.ck_conv; cs.conv_k = hp.conv_k;
-        if (p.run(T, st)) return -1;
         // a prefill chunk without checkpoints: the chunked rule on the matrix
-        // cores (delta_chunk.hip) over inputs prepared from the projections,
-        // then the gated RMSNorm (xj_cpu.c:215-217) as ssm_out's prep launch
+        // cores (delta_chunk.hip) over inputs prepared from the projections
+        // (after a GEMM the conv + SiLU in the same launch), then the gated
+        // RMSNorm (xj_cpu.c:215-217) as ssm_out's prep launch
         static const bool chunked_on = env_int("XJ_PREFILL_CHUNKED", 1) != 0;
         const int Sd = hp.s_k;
-        if (chunked_on && !pf && keep_n == 0 && T >= S->gemm_min && S->dwork && (Sd == 64 || Sd == 128) &&
-            hp.s_v == Sd && T <= S->s.max_batch) {
+        const bool chunked = chunked_on && !pf && keep_n == 0 && T >= S->gemm_min && S->dwork && (Sd == 64 || Sd == 128) &&
+                             hp.s_v == Sd && T <= S->s.max_batch;
+        p.raw_conv = chunked && p.gemm_ok(T);
+        if (p.run(T, st)) return -1;
+        if (chunked) {
             DeltaPrepArgs dp{};
             dp.qkv = S->qkv; dp.qkv_s = CD; dp.k_off = hp.key_dim; dp.v_off = 2 * hp.key_dim;
             dp.beta = S->beta; dp.beta_s = Hv; dp.alpha = S->alpha; dp.alpha_s = Hv; dp.dt = L.dt; dp.A = L.A;
             // kb / vb / u / g are free until the FFN: q, k, v [T][Hv][S], decay and beta [T][Hv]
             dp.q = S->kb; dp.k = S->vb; dp.v = S->u; dp.decay = S->g; dp.bt = S->g + (size_t)T * Hv;
             dp.T = T; dp.Hk = hp.h_k; dp.Hv = Hv; dp.S = Sd; dp.eps = hp.eps;
-            if (delta_prefill_prep_launch(dp, st) ||
+            dp.conv_state = L.conv; dp.conv_w = L.conv_w;
+            if ((p.raw_conv ? delta_conv_prep_launch(dp, CD, hp.conv_k, st) : delta_prefill_prep_launch(dp, st)) ||
                 delta_chunked_launch(Hv, Sd, T, 64, dp.q, dp.k, dp.v, dp.decay, dp.bt, 1.0f / sqrtf((float)Sd), L.ssm,
                                      S->o, S->dwork, st))
                 return -1;
@@ -799,12 +804,11 @@ int hip_rollback(xj_stage *s, int n_past, char *err, size_t errlen) {
 // reset succeeds.
 void hip_reset(xj_stage *s) {
     HStage *S = H(s);
-    hipError_t e = hipSuccess;
-    for (auto &L : S->L) {
-        if (!L.rec) continue;
-        if (e == hipSuccess) e = hipMemsetAsync(L.conv, 0, S->conv_n * 4, S->st);
-        if (e == hipSuccess) e = hipMemsetAsync(L.ssm, 0, S->ssm_n * 4, S->st);
-    }
+    // (one launch for every layer's states: 48 fills of a 4B stage took 0.25 ms)
+    hipError_t e = states_copy(S, S->st, [&](HLayer &L, const float *&, float *&cd, const float *&, float *&sd) {
+                       cd = L.conv;
+                       sd = L.ssm;
+                   }) ? hipErrorLaunchFailure : hipSuccess;
     const hipError_t e2 = hipStreamSynchronize(S->st);
     if (e == hipSuccess) e = e2;
     if (e == hipSuccess) e = hipGetLastError();

@@ -505,3 +505,23 @@ def test_chunk_attention_equals_single_steps(model_dir, H, Hkv, D, n_past, T):
     assert rel_l2(ya, yb) < 5e-5
     for s in (a, b):
         s.destroy()
+
+
+@pytest.mark.parametrize("conv_k,s_k,T", [(2, 64, 16), (3, 128, 23), (4, 128, 17), (8, 64, 65)])
+def test_chunk_conv_equals_single_steps(model_dir, conv_k, s_k, T):
+    """The conv + SiLU and L2 norms of a chunk in one launch (eight tokens per
+    wavefront, inputs before the chunk from the conv state, two value heads
+    per key head) and the state it leaves, over kernel sizes: hidden rows of a
+    chunk after five tokens and of two steps after it, against the same rows
+    fed one at a time."""
+    from conftest import synth_model
+    cfg = xp.TINY.with_(n_layer=4, conv_k=conv_k, s_k=s_k, h_k=2, h_v=4)
+    m = xp.Model(synth_model(model_dir, cfg, "tiny_c%d_%d" % (conv_k, s_k)))
+    a, b = (xp.HipStage(m, 0, 4, 128, 96, False) for _ in range(2))
+    rows = np.random.default_rng(T).standard_normal((T + 7, cfg.n_embd)).astype(np.float32)
+    a.forward(rows[:5].copy())
+    ya = np.concatenate([a.forward(rows[5:5 + T].copy())] + [a.forward(rows[i:i + 1].copy()) for i in (T + 5, T + 6)])
+    yb = np.concatenate([b.forward(rows[i:i + 1].copy()) for i in range(T + 7)])[5:]
+    assert rel_l2(ya, yb) < 5e-5
+    for s in (a, b):
+        s.destroy()
