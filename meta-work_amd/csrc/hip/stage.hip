@@ -48,9 +48,14 @@ struct WideBuf {
     int32_t n_cnt = 0;
 };
 
-// Chunks of at least kGemmMinT tokens take the matrix-core GEMM and the
-// chunked delta rule.
-constexpr int kGemmMinT = 16;
+// Chunks of at least kGemmMinT tokens take the matrix-core GEMM, of at least
+// kChunkMinT also the chunked delta rule and the matrix-core attention. Up to
+// ten tokens (two GEMV launches) a chunk keeps the single token's arithmetic
+// bit for bit, so that what a verification or its rollback leaves equals the
+// tokens fed alone; from eleven on that would take three launches, 52 us
+// against the GEMM's 21 us for 18432 x 2560 Q4_K at twelve. The DeltaNet step
+// kernel costs 2 us a token, the chunked rule 35 us with its preparation.
+constexpr int kGemmMinT = 11, kChunkMinT = 16;
 
 struct HLayer {
     bool rec = false;
@@ -101,7 +106,6 @@ struct HStage {
     int32_t *gcnt = nullptr;   // the GEMM's arrival counters (zero between launches)
     int32_t n_gcnt = 0;
     WideBuf wide;              // buffers of the wide GEMM (max_batch > 64)
-    int gemm_min = kGemmMinT;  // tokens from which a chunk takes the matrix-core path
     float2 *rope = nullptr;
     float *h_x = nullptr;            // pinned staging [max_batch][n_embd]
     int32_t *h_i = nullptr;          // pinned scalar
@@ -224,9 +228,8 @@ struct Gemv {
     bool prepared = false;
     explicit Gemv(uint8_t *xq, Profile *p = nullptr) : prof(p) { a.xq = xq; }
     Gemv(uint8_t *xq, Profile *p, float *tsc_, float *part_, int64_t part_floats_, int32_t *cnt_, int32_t n_cnt_,
-         uint8_t *hq_, const WideBuf *wide_, int gemm_min_)
-        : prof(p), tsc(tsc_), part(part_), part_floats(part_floats_), cnt(cnt_), n_cnt(n_cnt_), hq(hq_), wide(wide_),
-          gemm_min(gemm_min_) {
+         uint8_t *hq_, const WideBuf *wide_)
+        : prof(p), tsc(tsc_), part(part_), part_floats(part_floats_), cnt(cnt_), n_cnt(n_cnt_), hq(hq_), wide(wide_) {
         a.xq = xq;
     }
     Gemv &seg(const DevW &w, float *y, int ys, int epi) {
@@ -284,7 +287,6 @@ struct Gemv {
     bool hq_out = false;   // set by a GEMM run whose SwiGLU prep built the next input's hq
     bool raw_conv = false; // a GEMM run leaves the conv segment's projections as they are
     const WideBuf *wide = nullptr;
-    int gemm_min = kGemmMinT;
     // Chunks of at least kGemmMinT tokens take the matrix-core GEMM
     // (gemm.hip): the prep launch builds the T tokens' activations once, the
     // RMSNorm scale is applied per token after the dot products (as the GEMV
@@ -293,7 +295,7 @@ struct Gemv {
     // rows) and every other case keep the GEMV.
     bool gemm_ok(int T) const {
         static const bool on = env_int("XJ_PREFILL_GEMM", 1) != 0;
-        if (!on || T < gemm_min || prof || !tsc || !part || !cnt || !a.xq || !hq) return false;
+        if (!on || T < kGemmMinT || prof || !tsc || !part || !cnt || !a.xq || !hq) return false;
         if (a.pro != PRO_NONE && a.pro != PRO_RMSU && a.pro != PRO_SWIGLU && a.pro != PRO_GATED_RMS) return false;
         if (a.post.mode != POST_NONE && a.post.mode != POST_SWIGLU) return false;
         if (a.K % 256) return false;
@@ -490,7 +492,7 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
     HLayer &L = S->L[il - S->s.l0];
     const int E = hp.n_embd, FF = hp.n_ff;
     // every GEMV of the layer with the stage's prefill buffers
-    auto gemv = [&](uint8_t *xq) { return Gemv(xq, pf, S->tsc, S->gpart, S->gpart_floats, S->gcnt, S->n_gcnt, S->hq, &S->wide, S->gemm_min); };
+    auto gemv = [&](uint8_t *xq) { return Gemv(xq, pf, S->tsc, S->gpart, S->gpart_floats, S->gcnt, S->n_gcnt, S->hq, &S->wide); };
     auto rms_in = [&](Gemv &g, const float *w) {
         g.a.x = x; g.a.xs = E; g.a.pro = PRO_RMSU; g.a.pro_w = w; g.a.eps = hp.eps;
     };
@@ -509,7 +511,7 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
         // RMSNorm (xj_cpu.c:215-217) as ssm_out's prep launch
         static const bool chunked_on = env_int("XJ_PREFILL_CHUNKED", 1) != 0;
         const int Sd = hp.s_k;
-        const bool chunked = chunked_on && !pf && keep_n == 0 && T >= S->gemm_min && S->dwork && (Sd == 64 || Sd == 128) &&
+        const bool chunked = chunked_on && !pf && keep_n == 0 && T >= kChunkMinT && S->dwork && (Sd == 64 || Sd == 128) &&
                              hp.s_v == Sd && T <= S->s.max_batch;
         p.raw_conv = chunked && p.gemm_ok(T);
         if (p.run(T, st)) return -1;
@@ -576,7 +578,7 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
         q.seg(L.wo, x, E, EPI_ADD);
         // chunks on the matrix cores leave wo's input to its own prep launch; shorter ones, and those kept on
         // the GEMV's arithmetic, take the decode kernels, in slices of the split partials' scratch
-        if (!pf && T >= S->gemm_min) {
+        if (!pf && T >= kChunkMinT) {
             if (attn_chunk_launch(at, S->s.n_past, S->score_floats, st)) return -1;
             q.a.x = S->o; q.a.xs = Hq * D; q.a.pro = PRO_NONE;
         } else {
@@ -620,12 +622,16 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
     return dn.run(T, st);
 }
 
-// Every layer of the stage; inc: the stage's position counter advances by T
-// after the last of them.
-int enqueue_layers(HStage *S, float *x, int T, int keep_n, bool inc, hipStream_t st, Profile *pf = nullptr) {
-    for (int il = S->s.l0; il < S->s.l1; il++)
-        if (enqueue_layer(S, il, x, T, keep_n, inc && il + 1 == S->s.l1 ? S->npast : nullptr, st, pf)) return -1;
+// Layers [lo, hi) of the stage; inc: the position counter of its scratch
+// advances by T after the last of them.
+int enqueue_layer_range(HStage *S, int lo, int hi, float *x, int T, int keep_n, bool inc, hipStream_t st,
+                        Profile *pf = nullptr) {
+    for (int il = lo; il < hi; il++)
+        if (enqueue_layer(S, il, x, T, keep_n, inc && il + 1 == hi ? S->npast : nullptr, st, pf)) return -1;
     return 0;
+}
+int enqueue_layers(HStage *S, float *x, int T, int keep_n, bool inc, hipStream_t st, Profile *pf = nullptr) {
+    return enqueue_layer_range(S, S->s.l0, S->s.l1, x, T, keep_n, inc, st, pf);
 }
 
 // logits[t] = output . rmsnorm(x[t]) * output_norm; greedy partial keys into S->amax
@@ -848,7 +854,7 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
     S->score_floats = (int64_t)(mb < kAttnT ? mb : kAttnT) * hp.n_head * attn_splits(n_ctx) * (hp.head_dim + 2);
     S->scores = dalloc<float>(S, (size_t)S->score_floats, err, errlen);
     S->npast = dalloc<int32_t>(S, 1, err, errlen);
-    // prefill on the matrix cores (chunks of at least 16 tokens)
+    // prefill on the matrix cores
     S->tsc = dalloc<float>(S, mb, err, errlen);
     // every GEMM launch covers at most 2 sf + 2 h_v rows (gate|up, the DeltaNet in-projection)
     const int64_t grows = 2 * (int64_t)sf + 2 * (int64_t)hp.h_v;
@@ -898,8 +904,8 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
 }
 
 // A second set of scratch, for pieces of a prompt longer than the stage's
-// max_batch (chain_eval): the stage's weights, layer states, stream and
-// position counter.
+// max_batch (chain_eval): the stage's weights, layer states and stream, its
+// own position counter.
 static HStage *twin_new(HStage *S, int max_batch, char *err, size_t errlen) {
     HStage *T = new HStage();
     T->s = S->s;
@@ -912,7 +918,6 @@ static HStage *twin_new(HStage *S, int max_batch, char *err, size_t errlen) {
         delete T;
         return nullptr;
     }
-    T->npast = S->npast;
     return T;
 }
 static void twin_free(HStage *T) {
@@ -1227,6 +1232,7 @@ struct xjh_chain {
     int32_t *d_prompt = nullptr;
     int prompt_cap = 0;
     std::vector<hipEvent_t> ev_done, ev_taken;
+    hipStream_t half = nullptr;   // a single stage's later layers in a prompt of two short chunks
     // the app's sampler (xjh_chain_set_sampler): temperature, the uniform
     // numbers on the device, how many are drawn; the sampled decode graph
     float temp = 0.f;
@@ -1274,7 +1280,9 @@ extern "C" void xjh_chain_free(xjh_chain *c) {
     for (hipEvent_t e : c->ev_done) if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->ev_taken) if (e) (void)hipEventDestroy(e);
     if (c->d_prompt) (void)hipFree(c->d_prompt);
+    if (c->half) (void)hipStreamSynchronize(c->half);
     for (HStage *T : c->twins) twin_free(T);
+    if (c->half) (void)hipStreamDestroy(c->half);
     for (int32_t *p : {c->d_tokens, c->d_argmax, c->d_tok, c->d_hist, c->d_step, c->d_rbase, c->d_pick}) if (p) (void)hipFree(p);
     if (c->h_buf) (void)hipHostFree(c->h_buf);
     delete c;
@@ -1312,7 +1320,7 @@ extern "C" xjh_chain *xjh_chain_new(xj_stage **stages, int n, char *err, size_t 
         xjh_chain_free(c);
         return nullptr;
     }
-    const size_t nev = c->st.size();
+    const size_t nev = c->st.size() < 2 ? 2 : c->st.size();
     c->ev_done.assign(nev, nullptr);
     c->ev_taken.assign(nev, nullptr);
     for (size_t i = 0; i < nev; i++)
@@ -1324,7 +1332,7 @@ extern "C" xjh_chain *xjh_chain_new(xj_stage **stages, int n, char *err, size_t 
         }
     // stages whose chunks take the prefill GEMM get the pieces' scratch now, so
     // that the first long prompt does not pay for the allocations
-    if (c->mb >= kGemmMinT) (void)chain_twins(c);
+    if (c->mb >= kChunkMinT) (void)chain_twins(c);
     return c;
 }
 
@@ -1336,8 +1344,7 @@ static int chain_sync(xjh_chain *c, char *err, size_t errlen) {
 }
 
 // A prompt longer than max_batch, in pieces: of up to kPieceT tokens on the
-// stages' second scratch (chain_twins; from the 16 tokens on that take the
-// GEMM), else in chunks of max_batch. The stages are pipelined
+// stages' second scratch (chain_twins), else in chunks of max_batch. The stages are pipelined
 // (pipe/core/xj_net.c:561-604 pipelines a remote worker's half against the
 // host's): each stage runs on its own stream from its own hidden-state buffer,
 // so stage i works on piece k + 1 while stage i + 1 works on piece k. Stage
@@ -1351,45 +1358,58 @@ static int chain_finish(xjh_chain *c, int nl, int32_t *argmax, char *err, size_t
 // chain_finish collects the argmax of the nlog rows.
 static int chain_eval(xjh_chain *c, const int32_t *tokens, int n, int nlog, int keep, float *logits, int32_t *argmax,
                       char *err, size_t errlen, bool wait = true) {
-    const int B = c->mb, E = c->st[0]->s.m->hp.n_embd, np = (int)c->st.size();
+    const int B = c->mb, E = c->st[0]->s.m->hp.n_embd;
     if (!wait && (nlog < 1 || logits || n > B)) { snprintf(err, errlen, "asynchronous eval of one chunk with argmax only"); return -1; }
     if (n <= 0) { snprintf(err, errlen, "no tokens"); return -1; }
     if (keep && n > B) { snprintf(err, errlen, "verify batch %d exceeds max_batch %d", n, B); return -1; }
     static const bool overlap = env_int("XJ_CHAIN_OVERLAP", 1) != 0;
     HStage *head = c->st.back();
-    auto stream_of = [&](int i) { return overlap ? c->st[i]->st : c->stream; };
+    for (auto *S : c->st)
+        if (S->s.n_past + n > S->s.n_ctx) { snprintf(err, errlen, "context full (%d)", S->s.n_ctx); return -1; }
+    // prompts of one or two chunks too short for the matrix cores (max_batch <
+    // 16) stay in chunks, on the step kernels' arithmetic: what callers that
+    // feed such chunks themselves get, bit for bit
+    const bool wide = n > B && n >= kChunkMinT && (B >= kChunkMinT || n > 2 * B) && chain_twins(c);
+    // the pipeline's parts: layers [lo, hi) of a stage S on the scratch of R
+    struct Part { HStage *S, *R; int lo, hi; hipStream_t st; };
+    std::vector<Part> parts;
+    for (size_t i = 0; i < c->st.size(); i++) {
+        HStage *S = c->st[i];
+        parts.push_back(Part{S, wide ? c->twins[i] : S, S->s.l0, S->s.l1, overlap ? S->st : c->stream});
+    }
+    // two short chunks through a single stage: its later layers on the second
+    // scratch and a stream of their own, so that the second chunk's launches
+    // run beside the first's (0.8B, 16 tokens, max_batch 8: 5.0 -> 4.5 ms)
+    if (!wide && parts.size() == 1 && n > B && overlap && head->s.l1 - head->s.l0 > 1 && chain_twins(c) && B <= c->piece &&
+        (c->half || hipStreamCreateWithFlags(&c->half, hipStreamNonBlocking) == hipSuccess)) {
+        const int mid = (head->s.l0 + head->s.l1) / 2;
+        parts[0].hi = mid;
+        parts.push_back(Part{head, c->twins[0], mid, head->s.l1, c->half});
+    }
+    const int np = (int)parts.size();
     auto fail_sync = [&]() {
-        for (int i = 0; i < np; i++) (void)hipStreamSynchronize(stream_of(i));
+        for (auto &p : parts) (void)hipStreamSynchronize(p.st);
         for (auto *S : c->st) S->s.keep = 0;
         return -1;
     };
-    for (auto *S : c->st)
-        if (S->s.n_past + n > S->s.n_ctx) { snprintf(err, errlen, "context full (%d)", S->s.n_ctx); return -1; }
-    const bool wide = n > B && n >= kGemmMinT && chain_twins(c);
-    // stages whose own chunks are too short for the matrix cores (max_batch <
-    // 16) keep the GEMV's arithmetic for prompts up to twice that length, bit
-    // for bit that of the same tokens in chunks or steps
-    const int gemm_min = B < kGemmMinT && n < 2 * kGemmMinT ? 2 * kGemmMinT : kGemmMinT;
     if (n > c->prompt_cap) {
         if (c->d_prompt) (void)hipFree(c->d_prompt);
         c->d_prompt = nullptr, c->prompt_cap = 0;
         if (hipMalloc(&c->d_prompt, 4 * (size_t)n) != hipSuccess) { snprintf(err, errlen, "prompt allocation failed"); return -1; }
         c->prompt_cap = n;
     }
-    // the ids (synchronous copy from the caller's memory) and every stage's
+    // the ids (synchronous copy from the caller's memory) and every part's
     // starting position
     if (hipMemcpy(c->d_prompt, tokens, 4 * (size_t)n, hipMemcpyHostToDevice) != hipSuccess) {
         snprintf(err, errlen, "token upload failed"); return -1;
     }
-    for (int i = 0; i < np; i++) {
-        HStage *S = c->st[i];
-        *S->h_i = S->s.n_past;
-        if (hipMemcpyAsync(S->npast, S->h_i, 4, hipMemcpyHostToDevice, stream_of(i)) != hipSuccess ||
-            hipStreamSynchronize(stream_of(i)) != hipSuccess) {   // h_i is reused by later calls
+    for (auto &p : parts) {
+        *p.S->h_i = p.S->s.n_past;
+        if (hipMemcpyAsync(p.R->npast, p.S->h_i, 4, hipMemcpyHostToDevice, p.st) != hipSuccess ||
+            hipStreamSynchronize(p.st) != hipSuccess) {   // h_i is reused by later calls
             snprintf(err, errlen, "position upload failed"); return -1;
         }
     }
-    auto x_of = [&](int i) { return wide ? c->twins[i]->x : c->st[i]->x; };
     int Tp = 0;   // tokens of the last piece
     for (int k0 = 0; k0 < n; k0 += Tp) {
         const int left = n - k0;
@@ -1397,49 +1417,50 @@ static int chain_eval(xjh_chain *c, const int32_t *tokens, int n, int nlog, int 
         // the last piece keeps at least max_batch tokens (the rows a caller may ask for)
         else Tp = left <= c->piece ? left : left - c->piece < B ? c->piece / 2 : c->piece;
         for (int i = 0; i < np; i++) {
-            HStage *S = c->st[i];
-            hipStream_t st = stream_of(i);
-            float *x = x_of(i);
+            HStage *S = parts[i].S, *R = parts[i].R;
+            const hipStream_t st = parts[i].st;
             if (i == 0) {
-                // piece k0 into stage 0's buffer, once stage 1 has taken the previous one
+                // piece k0 into part 0's buffer, once part 1 has taken the previous one
                 if (np > 1 && k0 > 0 && hipStreamWaitEvent(st, c->ev_taken[1], 0) != hipSuccess) return fail_sync();
-                EmbedArgs ea{c->d_prompt + k0, S->tok_embd, x, Tp};
+                EmbedArgs ea{c->d_prompt + k0, S->tok_embd, R->x, Tp};
                 if (embed_launch(ea, st)) { snprintf(err, errlen, "embed launch failed"); return fail_sync(); }
             } else {
-                // this stage's previous piece is done with its buffer (same stream); the
-                // upstream stage's output of this piece is final
+                // this part's previous piece is done with its buffer (same stream); the
+                // upstream part's output of this piece is final
                 if (i + 1 < np && k0 > 0 && hipStreamWaitEvent(st, c->ev_taken[i + 1], 0) != hipSuccess) return fail_sync();
                 if (hipStreamWaitEvent(st, c->ev_done[i - 1], 0) != hipSuccess ||
-                    hipMemcpyAsync(x, x_of(i - 1), sizeof(float) * (size_t)Tp * E, hipMemcpyDeviceToDevice, st) != hipSuccess ||
+                    hipMemcpyAsync(R->x, parts[i - 1].R->x, sizeof(float) * (size_t)Tp * E, hipMemcpyDeviceToDevice, st) != hipSuccess ||
                     hipEventRecord(c->ev_taken[i], st) != hipSuccess) {
                     snprintf(err, errlen, "chunk hand-off failed"); return fail_sync();
                 }
             }
+            // the stage's bookkeeping with its first part, its position with the last
+            const bool first = i == 0 || parts[i - 1].S != S, last = i + 1 == np || parts[i + 1].S != S;
             int keep_n = 0;
-            HStage *R = S;   // the scratch the layers run on
-            if (wide) {
+            if (first && wide) {
                 if (reset_check(S, err, errlen)) return fail_sync();
-                R = c->twins[i];
-                R->L = S->L;   // checkpoint and snapshot buffers allocated since
-                R->gemm_min = gemm_min;
-                R->s.n_past = S->s.n_past;
                 S->s.keep = 0;
                 S->s.ck_start = S->s.n_past;
                 S->s.ck_T = 0;
-            } else {
+            } else if (first) {
                 if (keep) S->s.keep = Tp;
                 if (begin_forward(S, Tp, &keep_n, err, errlen)) return fail_sync();
             }
-            if (enqueue_layers(R, x, Tp, keep_n, true, st) || hipEventRecord(c->ev_done[i], st) != hipSuccess) {
+            if (R != S) {
+                R->L = S->L;   // checkpoint and snapshot buffers allocated since
+                R->s.n_past = S->s.n_past;
+            }
+            if (enqueue_layer_range(R, parts[i].lo, parts[i].hi, R->x, Tp, keep_n, true, st) ||
+                hipEventRecord(c->ev_done[i], st) != hipSuccess) {
                 snprintf(err, errlen, "layer launch failed"); return fail_sync();
             }
-            S->s.n_past += Tp;
-            if (k0 + Tp < n) S->s.keep = 0;
+            if (last) S->s.n_past += Tp;
+            if (last && k0 + Tp < n) S->s.keep = 0;
         }
     }
     const int T = n - (n - 1) / B * B;   // tokens of the last chunk of max_batch, the piece's last rows
-    const float *xl = x_of(np - 1) + (int64_t)(Tp - T) * E;
-    hipStream_t hs = stream_of(np - 1);
+    const float *xl = parts[np - 1].R->x + (int64_t)(Tp - T) * E;
+    hipStream_t hs = parts[np - 1].st;
     if (nlog > 0) {
         const int nl = nlog < T ? nlog : T;
         if (enqueue_head(head, xl + (int64_t)(T - nl) * E, nl, head->logits, hs) ||
@@ -1461,7 +1482,7 @@ static int chain_eval(xjh_chain *c, const int32_t *tokens, int n, int nlog, int 
         return 0;
     }
     for (int i = 0; i < np; i++) {
-        hipError_t e = hipStreamSynchronize(stream_of(i));
+        hipError_t e = hipStreamSynchronize(parts[i].st);
         if (e == hipSuccess) e = hipGetLastError();
         if (e != hipSuccess) { snprintf(err, errlen, "GPU error: %s", hipGetErrorString(e)); return fail_sync(); }
     }

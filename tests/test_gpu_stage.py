@@ -429,6 +429,28 @@ def test_prefill_chunk_with_checkpoints_rolls_back(tiny):
 
 
 
+@pytest.mark.parametrize("T", [11, 15])
+def test_short_chunk_on_the_gemm(tiny, T):
+    """Eleven to fifteen tokens take the GEMM with the decode's attention and
+    DeltaNet kernels (with checkpoints too): hidden rows against the same
+    tokens one at a time, and a rollback into the chunk. Bound: products 1e-6
+    apart (21- against 22-bit activations) round about 1e-6 / 2^-11 = 0.2% of
+    the fp16 keys and values the other way, each by 2^-11 of itself: 2e-5 of an
+    attention output, in two of the tiny model's eight layers, whose later
+    layers' norms and gates add up to a factor of a few (measured 7e-5)."""
+    m, L = tiny, tiny.hp.n_layer
+    toks = prompt_ids(m, T + 2, 600 + T)
+    a, b = xp.HipStage(m, 0, L, 64, 16, True), xp.HipStage(m, 0, L, 64, 16, True)
+    a.set_keep(T)
+    ya = a.forward(embed(m, toks[:T]))
+    yb = np.concatenate([b.forward(embed(m, toks[i:i + 1])) for i in range(T - 1)])
+    assert rel_l2(ya[:-1], yb) < 2e-4
+    a.rollback(T - 1)
+    assert rel_l2(a.forward(embed(m, toks[T:])), b.forward(embed(m, toks[T:]))) < 2e-4
+    for s in (a, b):
+        s.destroy()
+
+
 @pytest.mark.parametrize("T", [65, 96, 129, 200, 256])
 def test_wide_chunk_equals_chunks_of_64(tiny, T):
     """A chunk beyond 64 tokens takes the wide GEMM (256 x 128 tiles over
@@ -453,11 +475,11 @@ def test_wide_chunk_equals_chunks_of_64(tiny, T):
         s.destroy()
 
 
-@pytest.mark.parametrize("n,mb", [(40, 16), (200, 16), (31, 8), (33, 8), (1030, 64), (1601, 64)])
+@pytest.mark.parametrize("n,mb", [(40, 16), (200, 16), (16, 8), (17, 8), (1030, 64), (1601, 64)])
 def test_chain_prompt_pieces(tiny, n, mb):
     """A prompt beyond max_batch goes through the layers in pieces of up to
     1024 tokens (1030: 512 + 518, so that the last piece holds max_batch
-    rows; below 32 tokens with max_batch 8 on the GEMV): the logits of its
+    rows; two chunks of 8 stay chunks): the logits of its
     last rows are those of the vtable's chunks, one chain of two stages gives
     them bit for bit, and decoding continues from its state."""
     m, L = tiny, tiny.hp.n_layer
