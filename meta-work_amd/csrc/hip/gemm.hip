@@ -1,5 +1,5 @@
-// Multi-token dequant-GEMM on the matrix cores (gfx950), for prefill chunks of
-// 16..64 tokens (the reference's matmul, src/xiaoju-pipe/core/xj_cpu.c:36-54,
+// Multi-token dequant-GEMM on the matrix cores (gfx950), for chunks of up to 32
+// tokens (gemm_wide.hip takes more) (the reference's matmul, src/xiaoju-pipe/core/xj_cpu.c:36-54,
 // y[t][r] = sum_k deq(W_r)[k] x[t][k], over a whole chunk of tokens).
 //
 // Activations: the prep launch's hq records (xq.h): per token and 256-element
@@ -21,10 +21,8 @@
 // dequantized weights to ~1e-7 relative; the dot-product GEMV, whose
 // activations are 21-bit integers per 32-element group, agrees to ~1e-6.
 //
-// Work split: a row group of 128 rows per work-group of eight wavefronts.
-// Above 32 tokens a wavefront takes 32 rows (two 16-row tiles) x 32 tokens
-// (two 16-token tiles), the eight being four row pairs x two token halves;
-// otherwise 16 rows x every token. The units, a (row group, 256-element
+// Work split: a row group of 128 rows per work-group of eight wavefronts, 16
+// rows x every token each. The units, a (row group, 256-element
 // block) pair each over every segment of the launch, are dealt out in equal
 // contiguous ranges to one persistent work-group per CU. A work-group
 // requests a unit's weights and stages its activations of all tokens in LDS
@@ -63,7 +61,7 @@ __device__ __forceinline__ h8 cat8(h2 a, h2 b, h2 c, h2 d) {
 __device__ __forceinline__ h2 biased01(uint32_t w) { return as_h2(__builtin_amdgcn_perm(0x64646464u, w, 0x04010400u)); }
 __device__ __forceinline__ h2 biased23(uint32_t w) { return as_h2(__builtin_amdgcn_perm(0x64646464u, w, 0x04030402u)); }
 
-constexpr int kGemmMaxT = 64;
+constexpr int kGemmMaxT = 32;
 constexpr int kTokChunks = kHqBlk / 16;   // 16-byte chunks per token record
 constexpr int kRG = 128, kWaves = 8, kThreads = 64 * kWaves;   // rows and wavefronts per row group
 
@@ -299,20 +297,17 @@ __device__ __forceinline__ int wg_of(int u, int P, int G) { return ((u + 1) * G 
 template <bool Q6, int NTG>
 __device__ __forceinline__ void gemm_units(const GemmArgs &a, uint8_t *lds, int *last_sh_p, int wb, int w, int G,
                                            int P, int ub) {
-    // NTG 16-token column groups: above two, a wavefront takes two row tiles x
-    // two token tiles (four row pairs x two token halves), else one row tile x
-    // all of them
-    constexpr int RT = NTG > 2 ? 2 : 1, TT = NTG > 2 ? 2 : NTG;
+    // one row tile x NTG 16-token tiles per wavefront
+    constexpr int RT = 1, TT = NTG;
     int &last_sh = *last_sh_p;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, li = lane & 15, kq = lane >> 4;
     const int nb = a.nb;
     const int u0 = ub + w * P / G, u1 = ub + (w + 1) * P / G;
     uint8_t *const buf0 = lds, *const buf1 = lds + a.T * kHqBlk;
-    const int wrow = RT == 2 ? 32 * (wv >> 1) : 16 * wv;   // this wavefront's first row in the row group
-    const int tile0 = RT == 2 ? TT * (wv & 1) : 0;          // ... and first token tile
+    const int wrow = 16 * wv;   // this wavefront's first row in the row group
     int tok[TT];
 #pragma unroll
-    for (int tt = 0; tt < TT; tt++) tok[tt] = min(16 * (tile0 + tt) + li, a.T - 1);
+    for (int tt = 0; tt < TT; tt++) tok[tt] = min(16 * tt + li, a.T - 1);
     // row group g (global) -> segment s; this wavefront's rows (clamped so that
     // every load stays inside the weights; rows past N compute values that
     // are never stored)
@@ -374,12 +369,12 @@ __device__ __forceinline__ void gemm_units(const GemmArgs &a, uint8_t *lds, int 
             const int wf = wb + wg_of(first - ub, P, G), wl = wb + wg_of(first + nb - 1 - ub, P, G);
             const int r0 = (g - a.rg0[s]) * kRG;
             if (wf == wl) {
-                // lane holds rows rb + 16 rt + 4 kq + i of token 16 (tile0 + tt) + li
+                // lane holds rows rb + 16 rt + 4 kq + i of token 16 tt + li
 #pragma unroll
                 for (int rt = 0; rt < RT; rt++)
 #pragma unroll
                     for (int tt = 0; tt < TT; tt++) {
-                        const int t = 16 * (tile0 + tt) + li;
+                        const int t = 16 * tt + li;
 #pragma unroll
                         for (int i = 0; i < 4; i++) {
                             const int r = rb + 16 * rt + 4 * kq + i;
@@ -398,7 +393,7 @@ __device__ __forceinline__ void gemm_units(const GemmArgs &a, uint8_t *lds, int 
                 for (int rt = 0; rt < RT; rt++)
 #pragma unroll
                     for (int tt = 0; tt < TT; tt++) {
-                        const int t = 16 * (tile0 + tt) + li;
+                        const int t = 16 * tt + li;
                         if (t >= a.T) continue;
                         float *sp = slot + (int64_t)t * kRG + (rb - r0 + 16 * rt + 4 * kq);
                         const f4 y = acc[rt][tt] - accm[rt][tt];
@@ -591,19 +586,10 @@ int gemm_launch(const GemmArgs &in, int64_t part_floats, int n_cnt, hipStream_t 
     const bool q6 = a.type == XJ_Q6_K;
     const int ntg = (a.T + 15) / 16;
     if (a.n6) {
-        switch (ntg) {
-        case 1: launch_m<1>(a, lds, st); break;
-        case 2: launch_m<2>(a, lds, st); break;
-        case 3: launch_m<3>(a, lds, st); break;
-        default: launch_m<4>(a, lds, st); break;
-        }
+        ntg == 1 ? launch_m<1>(a, lds, st) : launch_m<2>(a, lds, st);
     } else {
-        switch (ntg) {
-        case 1: q6 ? launch_g<true, 1>(a, lds, st) : launch_g<false, 1>(a, lds, st); break;
-        case 2: q6 ? launch_g<true, 2>(a, lds, st) : launch_g<false, 2>(a, lds, st); break;
-        case 3: q6 ? launch_g<true, 3>(a, lds, st) : launch_g<false, 3>(a, lds, st); break;
-        default: q6 ? launch_g<true, 4>(a, lds, st) : launch_g<false, 4>(a, lds, st); break;
-        }
+        if (ntg == 1) q6 ? launch_g<true, 1>(a, lds, st) : launch_g<false, 1>(a, lds, st);
+        else q6 ? launch_g<true, 2>(a, lds, st) : launch_g<false, 2>(a, lds, st);
     }
     if (hipGetLastError() != hipSuccess) return -1;
     if (a.inc_ptr) {

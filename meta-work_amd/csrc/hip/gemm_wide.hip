@@ -1,4 +1,4 @@
-// Dequant-GEMM for long prompt pieces (65 tokens and more) on the matrix cores
+// Dequant-GEMM for prompt chunks and pieces of 33 tokens and more on the matrix cores
 // (gfx950): the products of gemm.hip (y[t][r] = sum_k deq(W_r)[k] x[t][k],
 // src/xiaoju-pipe/core/xj_cpu.c:36-54) for hundreds of tokens per launch, so
 // that a weight is decoded once per 128 tokens and wavefront pair.
@@ -51,8 +51,10 @@ typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef float f16v __attribute__((ext_vector_type(16)));
 typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 512;
+constexpr int kSkinnyT = 64;                      // tokens of the narrow kernel
 constexpr int kRows = 256, kToks = 128;          // a work-group's tile
 constexpr int kTokTiles = kToks / 32;
 constexpr int kStageB = 8192;                     // a 32-token tile's activations of 64 inner elements
@@ -71,6 +73,8 @@ struct Lds {
 };
 
 __device__ __forceinline__ f16v mfma(h8 a, h8 b, f16v c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+
+__device__ __forceinline__ f4 mfma16(h8 a, h8 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
 
 // Lane l: 16 (4) bytes at p to LDS offset off + 16 l (4 l); off is uniform over the wavefront.
 __device__ __forceinline__ void dma16(const uint8_t *p, uint32_t off) {
@@ -494,11 +498,271 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const WideArgs a
     }
 }
 
+// ------------------------------------------------------- 33..64 tokens --
+// The same products for a chunk of up to 64 tokens: a work-group takes few rows
+// (RT tiles of 16), all tokens and a range of the inner elements, which its
+// eight wavefronts share in contiguous chunks of 64 elements, each with sums of
+// its own for the whole tile on v_mfma_f32_16x16x32_f16 (tokens as rows of a
+// tile, weight rows as its columns). Every weight is decoded once; weights and
+// activations go straight to registers (the activation records' order serves
+// this operand too: group g's elements 8 kq .. + 7 are kstep kq & 1 of half
+// kq >> 1), no wavefront waits for another before the end, and only there the
+// sums meet, through LDS. Few rows (a 2560-row matrix is 160 tiles) are split
+// over the inner elements as well, the partial tiles added in order by the last
+// work-group to arrive.
+// It is bound by the latency of each chunk's activations at two wavefronts per
+// SIMD and by the 655 KB (K = 2560) of them that every work-group reads from
+// L2. 64 tokens: 18432 x 2560 Q4_K 37.4 -> 28.0 us, 2560 x 4096 Q4_K 24.0 ->
+// 13.5, 2560 x 9216 Q6_K 37.3 -> 27.8, against 128-row groups whose weights
+// were decoded twice and whose K ranges met through HBM. Its error against
+// float64 is the smaller too (0.9..1.6e-7 against 1.0..2.4e-7: shorter sums).
+// Below 33 tokens gemm.hip's kernels are as fast or faster (2560 x 9216 Q6_K at
+// 16: 15 against 20 us).
+template <bool Q6, int RT>
+struct SkW {
+    u2 q[RT][Q6 ? 3 : 1];   // Q4_K: the chunk's 8 bytes; Q6_K: low nibbles of its two groups, high bits
+    u4 hd[RT];              // Q4_K header, Q6_K scales
+    uint32_t d[RT];         // Q6_K
+};
+
+template <bool Q6, int RT, int NT>
+__global__ __launch_bounds__(512, 2) void gemm_skinny_kernel(const WideArgs a) {
+    extern __shared__ __align__(16) float red[];   // four wavefronts' sums
+    __shared__ int last_sh;
+    __shared__ float tsc[16 * NT];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), li = lane & 15, kq = lane >> 4;
+    const int nb = a.nb, rg = blockIdx.x / a.G, ks = blockIdx.x - rg * a.G;   // row group, split
+    const int C = 4 * nb, s0 = ks * C / a.G, s1 = (ks + 1) * C / a.G;
+    const int c0 = s0 + wv * (s1 - s0) / 8, c1 = s0 + (wv + 1) * (s1 - s0) / 8;   // this wavefront's chunks
+    const uint8_t *wp[RT];    // Q4_K: the row's blocks; Q6_K: its ql plane
+    int64_t b0[RT], NB[RT];
+#pragma unroll
+    for (int r = 0; r < RT; r++) {
+        const int tile = min(rg * RT + r, a.rt0[a.nseg] - 1);
+        int sg = 0;
+#pragma unroll
+        for (int k = 1; k < kGemmMaxSeg; k++) sg += k < a.nseg && tile >= a.rt0[k];
+        const int row = min((tile - a.rt0[sg]) * 16 + li, a.seg[sg].N - 1);
+        wp[r] = Q6 ? a.seg[sg].w : a.seg[sg].w + (int64_t)row * nb * 144;
+        b0[r] = (int64_t)row * nb;   // (Q6_K only)
+        NB[r] = (int64_t)a.seg[sg].N * nb;
+    }
+    auto load_w = [&](int c, SkW<Q6, RT> &w) {
+        const int blk = c >> 2, p = c & 3;
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            if constexpr (!Q6) {
+                const uint8_t *x = wp[r] + blk * 144;
+                w.q[r][0] = *(const u2 *)(x + 16 + 32 * p + 8 * kq);
+                w.hd[r] = *(const u4 *)x;
+            } else {
+                const int64_t b = b0[r] + blk;
+                const uint8_t *ql = wp[r] + b * 128 + 64 * (p >> 1) + 8 * kq;
+                w.q[r][0] = *(const u2 *)ql;
+                w.q[r][1] = *(const u2 *)(ql + 32);
+                w.q[r][2] = *(const u2 *)(wp[r] + NB[r] * 128 + b * 64 + 32 * (p >> 1) + 8 * kq);
+                w.hd[r][0] = *(const uint32_t *)(wp[r] + NB[r] * 192 + b * 16 + 4 * p);
+                w.d[r] = *(const uint16_t *)(wp[r] + NB[r] * 208 + b * 2);
+            }
+        }
+    };
+    // a chunk's activations of token tile t (16 tokens), two planes of its two groups
+    struct Act {
+        h8 h[2], l[2];
+        f4 ex;   // 2^e of tokens 16 t + 4 kq .. + 3
+    };
+    auto load_x = [&](int c, int t, Act &x) {
+        const int blk = c >> 2, p = c & 3;
+        const uint8_t *rec = a.wq + ((int64_t)(t >> 1) * nb + blk) * kWideRec;
+        const uint8_t *y = rec + p * kStageB + (kq & 1) * 2048 + ((kq >> 1) * 32 + 16 * (t & 1) + li) * 16;
+#pragma unroll
+        for (int g = 0; g < 2; g++) {
+            x.h[g] = *(const h8 *)(y + g * 4096);
+            x.l[g] = *(const h8 *)(y + g * 4096 + 1024);
+        }
+        x.ex = *(const f4 *)(rec + 4 * kStageB + 1024 + 4 * (16 * (t & 1) + 4 * kq));
+    };
+    f4 acc[RT][NT];
+#pragma unroll
+    for (int r = 0; r < RT; r++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[r][t] = f4{0.f, 0.f, 0.f, 0.f};
+    constexpr bool kAhead = RT * NT < 20;   // registers for the next chunk's weights
+    SkW<Q6, RT> w;
+    if (kAhead && c0 < c1) load_w(c0, w);
+    for (int c = c0; c < c1; c++) {
+        const int blk = c >> 2, p = c & 3;
+        if (!kAhead) load_w(c, w);
+        Act x[2];   // token tiles in turn, the one after next requested when one is done
+        load_x(c, 0, x[0]);
+        if constexpr (NT > 1) load_x(c, 1, x[1]);
+        // the weights' operands; the next chunk's weights are in flight from here
+        h8 A[RT][2], R[Q6 ? RT : 1][2], mB[Q6 ? 1 : RT];
+        float d[RT], dm[RT];
+#pragma unroll
+        for (int r = 0; r < RT; r++) {
+            if constexpr (!Q6) {
+                d[r] = xjd::f16_to_f32(w.hd[r][0] & 0xFFFFu);
+                dm[r] = -32.f * xjd::f16_to_f32(w.hd[r][0] >> 16);   // the group sums are stored / 32
+                const uint32_t lo = p < 2 ? w.hd[r][1] & 0x3F3F3F3Fu : (w.hd[r][3] & 0x0F0F0F0Fu) | ((w.hd[r][1] >> 2) & 0x30303030u);
+                const uint32_t sc2 = lo >> (16 * (p & 1));   // scales of groups 2 p and 2 p + 1 (xj_quant.h:49-52)
+#pragma unroll
+                for (int g = 0; g < 2; g++) {
+                    const h2 s2 = as_h2(__builtin_amdgcn_perm(0x64646464u, sc2, g ? 0x04010401u : 0x04000400u)) - h2{1024, 1024};
+                    const h2 n2 = s2 * h2{-1024, -1024};
+                    const uint32_t q0 = (g ? w.q[r][0][0] >> 4 : w.q[r][0][0]) & 0x0F0F0F0Fu,
+                                   q1 = (g ? w.q[r][0][1] >> 4 : w.q[r][0][1]) & 0x0F0F0F0Fu;
+                    A[r][g] = cat8(fma2(biased01(q0), s2, n2), fma2(biased23(q0), s2, n2), fma2(biased01(q1), s2, n2),
+                                   fma2(biased23(q1), s2, n2));
+                }
+                if (p == 0) {   // (uniform) the block's minimum terms with its first chunk
+                    const uint32_t m0 = w.hd[r][2] & 0x3F3F3F3Fu,
+                                   m1 = ((w.hd[r][3] >> 4) & 0x0F0F0F0Fu) | ((w.hd[r][2] >> 2) & 0x30303030u);
+                    const h2 b = {-1024, -1024};
+                    mB[r] = cat8(biased01(m0) + b, biased23(m0) + b, biased01(m1) + b, biased23(m1) + b);
+                }
+            } else {
+                d[r] = xjd::f16_to_f32(w.d[r]);
+#pragma unroll
+                for (int g = 0; g < 2; g++) {
+                    const int G = 2 * (p & 1) + g;   // low nibbles for G < 2, high bits at bit 2 G
+                    uint32_t q[2];
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        const uint32_t l4 = (p & 1 ? w.q[r][g][i] >> 4 : w.q[r][g][i]) & 0x0F0F0F0Fu;
+                        q[i] = l4 | (((w.q[r][2][i] >> (2 * G)) & 0x03030303u) << 4);
+                    }
+                    // scale 2 (2 p + g) + kq / 2: byte 2 g + kq / 2 of the chunk's word
+                    const _Float16 fs = (_Float16)(short)__builtin_amdgcn_sbfe((int)w.hd[r][0], 16 * g + 8 * (kq >> 1), 8);
+                    const h2 s2 = {fs, fs}, b = {-1056, -1056};
+                    const h2 x0 = biased01(q[0]) + b, x1 = biased23(q[0]) + b, x2 = biased01(q[1]) + b, x3 = biased23(q[1]) + b;
+                    const h2 f0 = x0 * s2, f1 = x1 * s2, f2 = x2 * s2, f3 = x3 * s2;
+                    A[r][g] = cat8(f0, f1, f2, f3);
+                    R[r][g] = cat8(fma2(x0, s2, -f0), fma2(x1, s2, -f1), fma2(x2, s2, -f2), fma2(x3, s2, -f3));
+                }
+            }
+        }
+        if (kAhead && c + 1 < c1) load_w(c + 1, w);
+#pragma unroll
+        for (int t = 0; t < NT; t++) {
+            const Act &y = x[t & 1];
+            f4 z[RT];
+#pragma unroll
+            for (int r = 0; r < RT; r++) z[r] = f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int g = 0; g < 2; g++) {   // the small terms first
+                if constexpr (Q6)
+#pragma unroll
+                    for (int r = 0; r < RT; r++) z[r] = mfma16(y.h[g], R[r][g], z[r]);
+#pragma unroll
+                for (int r = 0; r < RT; r++) z[r] = mfma16(y.l[g], A[r][g], z[r]);
+            }
+#pragma unroll
+            for (int g = 0; g < 2; g++)
+#pragma unroll
+                for (int r = 0; r < RT; r++) z[r] = mfma16(y.h[g], A[r][g], z[r]);
+#pragma unroll
+            for (int r = 0; r < RT; r++) acc[r][t] = acc[r][t] + y.ex * (z[r] * d[r]);
+            if constexpr (!Q6) {
+                if (p == 0) {   // eight groups' sums, hi in lanes kq = 0, lo in kq = 1
+                    const h8 v = *(const h8 *)(a.wq + ((int64_t)(t >> 1) * nb + blk) * kWideRec + 4 * kStageB + 512 * (kq & 1) +
+                                               (16 * (t & 1) + li) * 16);
+                    const h8 sx = kq < 2 ? v : h8{0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+                    for (int r = 0; r < RT; r++)
+                        acc[r][t] = acc[r][t] + y.ex * (mfma16(sx, mB[r], f4{0.f, 0.f, 0.f, 0.f}) * dm[r]);
+                }
+            }
+            if (t + 2 < NT) load_x(c, t + 2, x[t & 1]);
+        }
+    }
+    // the wavefronts' sums: 4..7 to 0..3, then the four copies to every thread's elements
+    f4 *rv = (f4 *)red;
+    constexpr int NV = RT * NT;   // f4 per lane
+    if (wv >= 4)
+#pragma unroll
+        for (int i = 0; i < NV; i++) rv[((wv - 4) * NV + i) * 64 + lane] = acc[i / NT][i % NT];
+    __syncthreads();
+    if (wv < 4)
+#pragma unroll
+        for (int i = 0; i < NV; i++) acc[i / NT][i % NT] = acc[i / NT][i % NT] + rv[(wv * NV + i) * 64 + lane];
+    __syncthreads();
+    if (wv < 4)
+#pragma unroll
+        for (int i = 0; i < NV; i++) rv[(wv * NV + i) * 64 + lane] = acc[i / NT][i % NT];
+    if (a.ss) {   // an RMSNorm input's scale per token, from the blocks' sums of x^2
+        if (tid < 16 * NT) {
+            const int t = min(tid, a.T - 1);
+            double sum = 0;
+            for (int b = 0; b < nb; b++) sum += a.ss[(int64_t)b * a.T + t];
+            tsc[tid] = 1.0f / sqrtf((float)(sum / a.K) + a.eps);
+        }
+    }
+    __syncthreads();
+    constexpr int NE = (NV * 64 + 511) / 512;   // f4 elements per thread: (tile pair i, lane)
+    f4 v[NE];
+#pragma unroll
+    for (int j = 0; j < NE; j++) {
+        const int e = min(tid + 512 * j, NV * 64 - 1);
+        v[j] = (rv[e] + rv[NV * 64 + e]) + (rv[2 * NV * 64 + e] + rv[3 * NV * 64 + e]);
+    }
+    if (a.G > 1) {
+        float *slot = a.part + (int64_t)blockIdx.x * (NV * 256);
+#pragma unroll
+        for (int j = 0; j < NE; j++) {
+            const int e = tid + 512 * j;
+            if (e >= NV * 64) continue;
+            store_sys2(slot + 4 * e, v[j][0], v[j][1]);
+            store_sys2(slot + 4 * e + 2, v[j][2], v[j][3]);
+        }
+        if (!xjd::arrive_last(a.cnt + rg, a.G, &last_sh)) return;
+#pragma unroll
+        for (int j = 0; j < NE; j++) v[j] = f4{0.f, 0.f, 0.f, 0.f};
+        for (int x = 0; x < a.G; x++) {
+            const float *src = a.part + (int64_t)(rg * a.G + x) * (NV * 256);
+            unsigned long long u[NE][2];
+#pragma unroll
+            for (int j = 0; j < NE; j++) {
+                const int e = min(tid + 512 * j, NV * 64 - 1);
+                u[j][0] = load_sys2(src + 4 * e);
+                u[j][1] = load_sys2(src + 4 * e + 2);
+            }
+#pragma unroll
+            for (int j = 0; j < NE; j++)
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    v[j][2 * k] += __uint_as_float((uint32_t)u[j][k]);
+                    v[j][2 * k + 1] += __uint_as_float((uint32_t)(u[j][k] >> 32));
+                }
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < NE; j++) {
+        const int e = tid + 512 * j, i = e >> 6, el = e & 63, r = i / NT, t = i - r * NT;
+        const int tile = rg * RT + r;
+        if (e >= NV * 64 || tile >= a.rt0[a.nseg]) continue;
+        int sgi = 0;
+#pragma unroll
+        for (int k = 1; k < kGemmMaxSeg; k++) sgi += k < a.nseg && tile >= a.rt0[k];
+        const GemmSeg &sg = a.seg[sgi];
+        const int row = (tile - a.rt0[sgi]) * 16 + (el & 15);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int tok = 16 * t + 4 * (el >> 4) + k;
+            if (row >= sg.N || tok >= a.T) continue;
+            float *yp = sg.y + (int64_t)tok * sg.ys + row;
+            const float y = a.ss ? v[j][k] * tsc[tok] : v[j][k];
+            *yp = sg.add ? *yp + y : y;
+        }
+    }
+}
+
 // The activations of 32 tokens and one 256-element block, in the order the
-// GEMM's lanes read them. A wavefront takes eight tokens, a lane four
+// GEMM's lanes read them. A wavefront takes four tokens, a lane four
 // consecutive elements k = 4 lane ..; the record is built in LDS and written
-// in one piece. Tokens past T are zero.
-__global__ __launch_bounds__(256) void wide_prep_kernel(const WidePrep a) {
+// in one piece. What it holds for tokens past T reaches their own sums only,
+// which are never stored.
+__global__ __launch_bounds__(512) void wide_prep_kernel(const WidePrep a) {
     __shared__ __align__(16) uint8_t rec[kWideRec];
     const int blk = blockIdx.x, tt = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int k = blk * 256 + 4 * lane;
@@ -506,24 +770,24 @@ __global__ __launch_bounds__(256) void wide_prep_kernel(const WidePrep a) {
     f4 pw = {1.f, 1.f, 1.f, 1.f};
     if (a.pro == PRO_RMSU) pw = *(const f4 *)(a.pro_w + k);
     if (a.pro == PRO_GATED_RMS) pw = *(const f4 *)(a.pro_w + k % a.group);
-    f4 xr[8], zr[8];
+    f4 xr[4], zr[4];
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int t = min(tt * 32 + wv * 8 + j, a.T - 1);
+    for (int j = 0; j < 4; j++) {
+        const int t = min(tt * 32 + wv * 4 + j, a.T - 1);
         xr[j] = *(const f4 *)(a.x + (int64_t)t * a.xs + k);
         if (a.x2) zr[j] = *(const f4 *)(a.x2 + (int64_t)t * a.x2s + k);
     }
 #pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int tl = wv * 8 + j, t = tt * 32 + tl;
-        const bool in = t < a.T;
+    for (int j = 0; j < 4; j++) {
+        const int tl = wv * 4 + j, t = tt * 32 + tl;
+        if (t >= a.T) break;   // uniform over the wavefront
         f4 v = xr[j];
         if (a.pro == PRO_RMSU) {
             double ss = 0;
 #pragma unroll
             for (int i = 0; i < 4; i++) ss += (double)v[i] * v[i];
             ss = xjd::wave_sum_d(ss);
-            if (lane == 0 && in) a.ss[(int64_t)blk * a.T + t] = ss;
+            if (lane == 0) a.ss[(int64_t)blk * a.T + t] = ss;
             v = v * pw;
         } else if (a.pro == PRO_SWIGLU) {
 #pragma unroll
@@ -537,7 +801,6 @@ __global__ __launch_bounds__(256) void wide_prep_kernel(const WidePrep a) {
 #pragma unroll
             for (int i = 0; i < 4; i++) v[i] = v[i] * sc * pw[i] * xjd::silu(zr[j][i]);
         }
-        if (!in) v = f4{0.f, 0.f, 0.f, 0.f};
         const float m = xjd::wave_max(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
         int E = 0;
         (void)frexpf(m, &E);   // m < 2^E
@@ -566,7 +829,7 @@ __global__ __launch_bounds__(256) void wide_prep_kernel(const WidePrep a) {
     }
     __syncthreads();
     uint8_t *dst = a.wq + ((int64_t)tt * a.nb + blk) * kWideRec;
-    for (int i = tid; i < (4 * kStageB + 1024 + 128) / 16; i += 256) ((u4 *)dst)[i] = ((const u4 *)rec)[i];
+    for (int i = tid; i < (4 * kStageB + 1024 + 128) / 16; i += 512) ((u4 *)dst)[i] = ((const u4 *)rec)[i];
 }
 
 int wide_cus() {
@@ -588,14 +851,56 @@ int launch_w(const WideArgs &a, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+template <bool Q6, int RT, int NT>
+int launch_s3(const WideArgs &a, int grid, hipStream_t st) {
+    constexpr int lds = 4 * RT * NT * 64 * 16;
+    static const bool raised = hipFuncSetAttribute((const void *)gemm_skinny_kernel<Q6, RT, NT>,
+                                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds) == hipSuccess;
+    if (!raised) return -1;
+    hipLaunchKernelGGL((gemm_skinny_kernel<Q6, RT, NT>), dim3(grid), dim3(512), lds, st, a);
+    return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+template <bool Q6, int RT>
+int launch_s2(const WideArgs &a, int grid, hipStream_t st) {
+    return a.T <= 48 ? launch_s3<Q6, RT, 3>(a, grid, st) : launch_s3<Q6, RT, 4>(a, grid, st);
+}
+
+// Row tiles per work-group and splits of the inner elements: the least cost in
+// units of a wavefront's chunk: the rounds of work-groups over the CUs times the
+// chunks' row tiles (dearer with the token tiles) and a fixed part, and for a
+// split the adding. Measured best at 37 and 64 tokens: 18432 x 2560 five tiles
+// unsplit (28.0 us at 64; three tiles 36.1), 12352 x 2560 four (22.4; five
+// 26.0), 2560 x 4096 two in three splits (13.5; one unsplit 17.7), 2560 x 9216
+// Q6_K two in three (27.8; three in four 31.0).
+struct SkPlan {
+    int rt, ks;
+};
+SkPlan skinny_plan(bool q6, int tiles, int nb, int nt) {
+    SkPlan best{1, 1};
+    double lo = 1e30;
+    for (int rt = 1; rt <= (q6 ? 3 : 5); rt++)
+        for (int ks = 1; ks <= 16 && ks <= nb; ks++) {
+            const int wgs = (tiles + rt - 1) / rt * ks, rounds = (wgs + wide_cus() - 1) / wide_cus();
+            if (ks > 1 && rounds > 1) break;
+            const int cw = ((4 * nb + ks - 1) / ks + 7) / 8;
+            const double c = rounds * ((rt * (0.5 + 0.5 * nt) + 1.5) * cw + 4.0) + (ks > 1 ? 6.0 + 0.5 * rt * ks : 0.0);
+            if (c < lo) lo = c, best = SkPlan{rt, ks};
+        }
+    return best;
+}
+
 }  // namespace
 
 size_t wide_wq_bytes(int K, int T) {
     return (size_t)((T + kToks - 1) / kToks) * kTokTiles * (K / 256) * kWideRec;
 }
-int64_t wide_part_floats() { return (int64_t)2 * wide_cus() * kRows * kToks; }
+int64_t wide_part_floats(int T) {
+    const int64_t skinny = (int64_t)wide_cus() * 5 * 4 * 256;
+    return T <= kSkinnyT ? skinny : std::max(skinny, (int64_t)2 * wide_cus() * kRows * kToks);
+}
 int wide_counters(int64_t rows, int T) {
-    return (int)((rows + 32 * kGemmMaxSeg + kRows - 1) / kRows + 1) * ((T + kToks - 1) / kToks);
+    const int64_t tiles = ((rows + 32 * kGemmMaxSeg + kRows - 1) / kRows + 1) * ((T + kToks - 1) / kToks);
+    return (int)(T <= kSkinnyT ? wide_cus() : std::max<int64_t>(wide_cus(), tiles));
 }
 
 int wide_prep_launch(const WidePrep &in, hipStream_t st) {
@@ -608,7 +913,7 @@ int wide_prep_launch(const WidePrep &in, hipStream_t st) {
     if (a.pro == PRO_GATED_RMS && ((a.group != 64 && a.group != 128) || !a.pro_w || ((uintptr_t)a.pro_w & 15))) return -1;
     if (a.pro != PRO_NONE && a.pro != PRO_RMSU && !two) return -1;
     a.nb = a.K / 256;
-    hipLaunchKernelGGL(wide_prep_kernel, dim3(a.nb, (a.T + 31) / 32), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(wide_prep_kernel, dim3(a.nb, (a.T + 31) / 32), dim3(512), 0, st, a);
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -618,12 +923,28 @@ int gemm_wide_launch(const WideArgs &in, int64_t part_floats, int n_cnt, hipStre
         !a.wq || !a.part || !a.cnt || ((uintptr_t)a.wq & 15))
         return -1;
     a.rt0[0] = 0;
+    const int tr = a.T <= kSkinnyT ? 16 : 32;   // rows per tile
     for (int i = 0; i < a.nseg; i++) {
         if (!a.seg[i].w || !a.seg[i].y || a.seg[i].N < 1 || ((uintptr_t)a.seg[i].w & 15)) return -1;
-        a.rt0[i + 1] = a.rt0[i] + (a.seg[i].N + 31) / 32;
+        a.rt0[i + 1] = a.rt0[i] + (a.seg[i].N + tr - 1) / tr;
     }
     for (int i = a.nseg + 1; i <= kGemmMaxSeg; i++) a.rt0[i] = a.rt0[a.nseg];
     a.nb = a.K / 256;
+    if (a.T <= kSkinnyT) {
+        const bool q6 = a.type == XJ_Q6_K;
+        const int nt = a.T <= 48 ? 3 : 4;
+        const SkPlan p = skinny_plan(q6, a.rt0[a.nseg], a.nb, nt);
+        const int groups = (a.rt0[a.nseg] + p.rt - 1) / p.rt;
+        a.G = p.ks;
+        if (p.ks > 1 && (groups > n_cnt || (int64_t)groups * p.ks * p.rt * nt * 256 > part_floats)) return -1;
+        switch (p.rt) {
+        case 1: return q6 ? launch_s2<true, 1>(a, groups * p.ks, st) : launch_s2<false, 1>(a, groups * p.ks, st);
+        case 2: return q6 ? launch_s2<true, 2>(a, groups * p.ks, st) : launch_s2<false, 2>(a, groups * p.ks, st);
+        case 3: return q6 ? launch_s2<true, 3>(a, groups * p.ks, st) : launch_s2<false, 3>(a, groups * p.ks, st);
+        case 4: return launch_s2<false, 4>(a, groups * p.ks, st);
+        default: return launch_s2<false, 5>(a, groups * p.ks, st);
+        }
+    }
     a.nrg = (a.rt0[a.nseg] + 7) / 8;
     const int tiles = a.nrg * ((a.T + kToks - 1) / kToks);
     a.P = (int64_t)tiles * a.nb;

@@ -168,7 +168,7 @@ int inc_launch(int32_t *p, int32_t by, hipStream_t st);
 int gemm_max_tokens();
 int gemm_launch(const GemmArgs &a, int64_t part_floats, int n_cnt, hipStream_t st);
 
-// The same products for long prompt pieces (gemm_wide.hip). Activations: one
+// The same products for 33 tokens and more (gemm_wide.hip). Activations: one
 // record of kWideRec bytes per 32 tokens and 256-element block (tile-major,
 // then block): for each stage of 64 inner elements the f16 planes hi and lo
 // in MFMA operand order (32 KB in all), then the group sums of hi + lo / 32
@@ -191,16 +191,17 @@ struct WideArgs {
     int32_t nseg;
     GemmSeg seg[kGemmMaxSeg];
     const double *ss; float eps;    // optional: y[t][r] = sum * rms scale of token t (from the sums of x^2)
-    float *part;                    // wide_part_floats() floats
+    float *part;                    // wide_part_floats(T) floats
     int32_t *cnt;                   // wide_counters(rows, T) ints, zero before the first launch, left zero
     // set by gemm_wide_launch
-    int32_t rt0[kGemmMaxSeg + 1];   // first 32-row tile of each segment (prefix)
-    int32_t nb, nrg, G;             // blocks per row, row groups, work-groups
+    int32_t rt0[kGemmMaxSeg + 1];   // first 32-row (up to 64 tokens: 16-row) tile of each segment (prefix)
+    int32_t nb, nrg, G;             // blocks per row, row groups, work-groups (up to 64 tokens: splits of K)
     int64_t P;                      // units
 };
 size_t wide_wq_bytes(int K, int T);
-int64_t wide_part_floats();
-int wide_counters(int64_t rows, int T);   // rows in all segments of a launch
+// capacities for launches of up to T tokens (rows in all segments)
+int64_t wide_part_floats(int T);
+int wide_counters(int64_t rows, int T);
 int wide_prep_launch(const WidePrep &a, hipStream_t st);
 int gemm_wide_launch(const WideArgs &a, int64_t part_floats, int n_cnt, hipStream_t st);
 

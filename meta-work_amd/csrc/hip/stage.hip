@@ -303,10 +303,10 @@ struct Gemv {
         for (int i = 0; i < a.nseg; i++) any = any || a.seg[i].type == XJ_Q4_K || a.seg[i].type == XJ_Q6_K;
         return any;
     }
-    // Chunks beyond the 64 tokens of a gemm.hip launch take the wide GEMM
-    // (gemm_wide.hip; 18432 x 2560 Q4_K, T = 128: 45 us against two launches of
-    // 37 us, T = 1024: 232 us against 16), which reads the plain input: a
-    // caller whose input would be prepared asks first and passes x instead.
+    // Chunks beyond the 32 tokens of a gemm.hip launch take gemm_wide.hip
+    // (18432 x 2560 Q4_K, T = 64: 28 us against 37 us in one launch of 64, T =
+    // 1024: 232 us against 16 such), which reads the plain input: a caller whose
+    // input would be prepared asks first and passes x instead.
     bool wide_ok(int T) const {
         auto al = [](const void *p, int32_t s) { return !((uintptr_t)p & 15) && !(s & 3); };
         if (T <= gemm_max_tokens() || !gemm_ok(T) || prepared || !wide || !wide->wq || !a.x || !al(a.x, a.xs)) return false;
@@ -606,7 +606,7 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
     Gemv dn = gemv(S->xq_ff);
     dn.a.x = S->g; dn.a.xs = FF; dn.a.x2 = S->u; dn.a.x2s = FF; dn.a.pro = PRO_SWIGLU;
     dn.seg(L.ffn_down, x, E, EPI_ADD);
-    const bool wide = f.wide_ok(T) && dn.wide_ok(T);   // silu(gate) * up formed by down's own prep
+    const bool wide = dn.wide_ok(T);   // silu(gate) * up formed by down's own prep
     if (!h && !wide) f.post(POST_SWIGLU, S->xq_ff, S->cnt_grp);
     if (f.run(T, st)) return -1;
     if (!wide) dn.a.x = dn.a.x2 = nullptr, dn.a.pro = PRO_NONE;
@@ -869,7 +869,7 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
         WideBuf &w = S->wide;
         w.wq = dalloc<uint8_t>(S, wide_wq_bytes((int)(sf / 256 * 256), (int)mb), err, errlen);
         w.ss = dalloc<double>(S, mb * (E / 256), err, errlen);
-        w.part_floats = wide_part_floats();
+        w.part_floats = wide_part_floats((int)mb);
         w.part = dalloc<float>(S, (size_t)w.part_floats, err, errlen);
         w.n_cnt = wide_counters(grows, (int)mb);
         w.cnt = dalloc<int32_t>(S, (size_t)w.n_cnt, err, errlen);
@@ -980,7 +980,7 @@ extern "C" uint64_t xj_hip_stage_state_bytes(const xj_model *m, int l0, int l1, 
          4ull * gemm_counters(grows) + (uint64_t)max_batch * hq_stride((int)scratch_floats(hp));
     if (max_batch > gemm_max_tokens())
         b += wide_wq_bytes((int)(scratch_floats(hp) / 256 * 256), max_batch) + 8ull * max_batch * (hp.n_embd / 256) +
-             4ull * wide_part_floats() + 4ull * wide_counters(grows, max_batch);
+             4ull * wide_part_floats(max_batch) + 4ull * wide_counters(grows, max_batch);
     bool rec = false;
     for (int il = l0; il < l1 && il < (int)hp.n_layer; il++) rec = rec || m->layers[il].recurrent;
     if (rec) b += delta_chunked_work_bytes(hp.h_v, hp.s_k, max_batch, 64);
@@ -2413,9 +2413,42 @@ extern "C" int xjh_gemv_noalloc(uint32_t type, const void *dw, int64_t n_rows, i
     return ops_done(err, errlen);
 }
 
-// Prepared activations of T tokens (prep launch) and the matrix-core GEMM.
+// Activations of T tokens (prep launch) and the matrix-core GEMM of their count.
 static int gemm_enqueue(uint32_t type, const void *dw, int64_t n_rows, int64_t k, const float *x, int T, float *y, int add,
                         hipStream_t st) {
+    auto grow = [](auto *&p, size_t &cap, size_t need) {   // grown on demand; the per-op entries are synchronous on one stream
+        if (need <= cap) return true;
+        if (p) (void)hipFree(p);
+        p = nullptr, cap = 0;
+        if (hipMalloc(&p, need * sizeof(*p)) != hipSuccess) return false;
+        cap = need;
+        return true;
+    };
+    if (T > gemm_max_tokens() && !((uintptr_t)x & 15)) {
+        static uint8_t *wq = nullptr;
+        static float *part = nullptr;
+        static int32_t *cnt = nullptr;
+        static size_t wq_cap = 0, part_cap = 0, cnt_cap = 0;
+        const size_t cneed = (size_t)wide_counters(n_rows, T);
+        const bool fresh = cneed > cnt_cap;   // zero once; the kernel leaves them zero
+        if (!grow(wq, wq_cap, wide_wq_bytes((int)k, T)) || !grow(part, part_cap, (size_t)wide_part_floats(T)) ||
+            !grow(cnt, cnt_cap, cneed) || (fresh && hipMemsetAsync(cnt, 0, cneed * 4, st) != hipSuccess))
+            return -1;
+        WidePrep p{};
+        p.x = x; p.xs = (int32_t)k; p.pro = PRO_NONE; p.wq = wq; p.K = (int32_t)k; p.T = T;
+        WideArgs g{};
+        g.type = type; g.K = (int32_t)k; g.T = T; g.wq = wq; g.part = part; g.cnt = cnt;
+        g.nseg = 1;
+        g.seg[0] = GemmSeg{(const uint8_t *)dw, (int32_t)n_rows, y, (int32_t)n_rows, add};
+        return wide_prep_launch(p, st) ? -1 : gemm_wide_launch(g, (int64_t)part_cap, (int)cnt_cap, st);
+    }
+    if (T > gemm_max_tokens()) {   // x not 16-byte aligned
+        for (int t0 = 0; t0 < T; t0 += gemm_max_tokens()) {
+            const int n = T - t0 < gemm_max_tokens() ? T - t0 : gemm_max_tokens();
+            if (gemm_enqueue(type, dw, n_rows, k, x + (int64_t)t0 * k, n, y + (int64_t)t0 * n_rows, add, st)) return -1;
+        }
+        return 0;
+    }
     static uint8_t *xq = nullptr, *hq = nullptr;   // grown on demand; the per-op entries are synchronous on one stream
     static float *part = nullptr;
     static int32_t *cnt = nullptr;
@@ -2423,30 +2456,10 @@ static int gemm_enqueue(uint32_t type, const void *dw, int64_t n_rows, int64_t k
     const int64_t xs = xq_off((int)k).stride, hs = hq_stride((int)k);
     const size_t need = (size_t)T * xs, hneed = (size_t)T * hs, pneed = (size_t)gemm_part_floats(n_rows, T),
                  cneed = (size_t)gemm_counters(n_rows);
-    if (need > xq_cap) {
-        if (xq) (void)hipFree(xq);
-        xq = nullptr, xq_cap = 0;
-        if (hipMalloc(&xq, need) != hipSuccess) return -1;
-        xq_cap = need;
-    }
-    if (hneed > hq_cap) {
-        if (hq) (void)hipFree(hq);
-        hq = nullptr, hq_cap = 0;
-        if (hipMalloc(&hq, hneed) != hipSuccess) return -1;
-        hq_cap = hneed;
-    }
-    if (pneed > part_cap) {
-        if (part) (void)hipFree(part);
-        part = nullptr, part_cap = 0;
-        if (hipMalloc(&part, pneed * 4) != hipSuccess) return -1;
-        part_cap = pneed;
-    }
-    if (cneed > cnt_cap) {   // zero once; the kernel leaves them zero
-        if (cnt) (void)hipFree(cnt);
-        cnt = nullptr, cnt_cap = 0;
-        if (hipMalloc(&cnt, cneed * 4) != hipSuccess || hipMemsetAsync(cnt, 0, cneed * 4, st) != hipSuccess) return -1;
-        cnt_cap = cneed;
-    }
+    const bool fresh = cneed > cnt_cap;   // zero once; the kernel leaves them zero
+    if (!grow(xq, xq_cap, need) || !grow(hq, hq_cap, hneed) || !grow(part, part_cap, pneed) || !grow(cnt, cnt_cap, cneed) ||
+        (fresh && hipMemsetAsync(cnt, 0, cneed * 4, st) != hipSuccess))
+        return -1;
     GArgs p{};
     p.x = x; p.xs = (int32_t)k; p.pro = PRO_NONE; p.xq = xq; p.K = (int32_t)k; p.T = T; p.hq = hq;
     if (prep_launch(p, st)) return -1;
@@ -2457,12 +2470,14 @@ static int gemm_enqueue(uint32_t type, const void *dw, int64_t n_rows, int64_t k
     return gemm_launch(g, (int64_t)part_cap, (int)cnt_cap, st);
 }
 
+constexpr int kGemmEntryT = 64;   // tokens of one xjh_gemm call
+
 extern "C" int xjh_gemm(uint32_t type, const void *dw, int64_t n_rows, int64_t k, const float *x, int T, float *y, int add,
                         char *err, size_t errlen) {
     if (!ops_stream()) return -1;
-    if ((type != XJ_Q4_K && type != XJ_Q6_K) || T < 1 || T > gemm_max_tokens() || n_rows < 1 || n_rows > INT32_MAX ||
+    if ((type != XJ_Q4_K && type != XJ_Q6_K) || T < 1 || T > kGemmEntryT || n_rows < 1 || n_rows > INT32_MAX ||
         k < 256 || k % 256) {
-        snprintf(err, errlen, "unsupported GEMM shape/type (Q4_K or Q6_K, K %% 256 == 0, 1 <= T <= %d)", gemm_max_tokens());
+        snprintf(err, errlen, "unsupported GEMM shape/type (Q4_K or Q6_K, K %% 256 == 0, 1 <= T <= %d)", kGemmEntryT);
         return -1;
     }
     if (gemm_enqueue(type, dw, n_rows, k, x, T, y, add, g_stream)) { snprintf(err, errlen, "GEMM launch failed"); return -1; }
@@ -2472,7 +2487,7 @@ extern "C" int xjh_gemm(uint32_t type, const void *dw, int64_t n_rows, int64_t k
 extern "C" double xjh_gemm_time(uint32_t type, void *const *dws, int n_copies, int64_t n_rows, int64_t k, const float *x,
                                 int T, float *y, int iters, char *err, size_t errlen) {
     if (!ops_stream()) return -1;
-    if ((type != XJ_Q4_K && type != XJ_Q6_K) || T < 1 || T > gemm_max_tokens() || k < 256 || k % 256) {
+    if ((type != XJ_Q4_K && type != XJ_Q6_K) || T < 1 || T > kGemmEntryT || k < 256 || k % 256) {
         snprintf(err, errlen, "unsupported GEMM shape/type"); return -1;
     }
     hipEvent_t e0, e1;

@@ -72,3 +72,27 @@ def test_gemm_rejects_unsupported():
     q8 = xp.DevWeight(xp.Q8_0, _weights(xp.Q8_0, 64, 256, 4), 64, 256)
     with pytest.raises(xp.XjError):
         xp.gemm(q8, np.zeros((16, 256), np.float32))
+
+
+@pytest.mark.parametrize("t,rows,k", [
+    (xp.Q4_K, 18432, 256),     # more row tiles than work-groups: five per work-group, K unsplit
+    (xp.Q4_K, 2560, 4096),     # two row tiles per work-group, K in three splits
+    (xp.Q4_K, 1009, 2560),     # a last row tile of one row
+    (xp.Q6_K, 2560, 9216),     # Q6_K, K in three splits of 48 chunks
+    (xp.Q6_K, 33, 512),        # eight chunks over eight wavefronts and two splits
+    (xp.Q4_K, 5, 256),         # four chunks: wavefronts without work
+])
+@pytest.mark.parametrize("T", [33, 48, 49, 63])
+def test_narrow_gemm_edges(t, rows, k, T):
+    """33 to 64 tokens: edges of the token tiles (three up to 48, else four),
+    row tiles and splits of the inner elements. Activations of 22 bits, exact
+    products and fp32 sums: 1.7e-7 of float64 measured, four times that
+    allowed; the residual-add form adds to what is there."""
+    blob = _weights(t, rows, k, 3000 + rows + k)
+    xs = xp.fill_normal(T * k, 191 + T, 1.0).reshape(T, k)
+    w = xp.DevWeight(t, blob, rows, k)
+    got = xp.gemm(w, xs)
+    ref64 = xs.astype(np.float64) @ orc.dequant_rows(t, blob, rows, k).astype(np.float64).T
+    assert rel_l2(got, ref64) < 7e-7
+    base = xp.fill_normal(T * rows, 19, 1.0).reshape(T, rows)
+    assert np.array_equal(xp.gemm(w, xs, add_to=base), base + got)
