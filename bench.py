@@ -84,8 +84,8 @@ def decode_run(cfg, name, n_prompt, steps, warmup, seed):
     log(f"{name}: uploaded in {time.time() - t:.1f} s ({xp.tune_note()})")
     ch = xp.Chain([st])
     prompt = np.random.default_rng(seed).integers(0, hp.n_vocab, n_prompt).astype(np.int32)
-    # warm-up of the prefill path over two chunks (so the pipelined parts' scratch
-    # is allocated and their kernels loaded), then a fresh stage state
+    # warm-up of the prefill path over two chunks' tokens (so that its kernels
+    # are loaded), then a fresh stage state
     ch.eval(prompt[:128])
     ch.reset()
     t = time.perf_counter()

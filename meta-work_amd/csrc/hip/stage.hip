@@ -1258,6 +1258,7 @@ static bool chain_twins(xjh_chain *c) {
             for (HStage *t : c->twins) twin_free(t);
             c->twins.clear();
             c->piece = -1;
+            (void)hipGetLastError();   // the failed allocation must not fail the launches that follow
             return false;
         }
         c->twins.push_back(T);

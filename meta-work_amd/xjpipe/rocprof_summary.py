@@ -61,7 +61,7 @@ def trace(d):
     # token); steps are the spans between consecutive argmax launches that
     # hold single-token GEMVs only
     ends = [i for i, r in enumerate(rows) if r["Kernel_Name"].startswith("xjk::finalize")]
-    several = re.compile(r"xjk::(gemv_kernel|gemv_cu_kernel)<[2-9],|xjk::(gemm_mfma|dc_|conv_silu|prep_kernel)")
+    several = re.compile(r"xjk::(gemv_kernel|gemv_cu_kernel)<[2-9],|xjk::(gemm_mfma|gemm_wide|gemm_skinny|wide_prep|attn_chunk|delta_conv_prep|conv_tail|dc_|conv_silu|prep_kernel)")
     steps = [rows[a + 1:b + 1] for a, b in zip(ends, ends[1:])
              if any(_gemv1(r["Kernel_Name"]) for r in rows[a + 1:b + 1])
              and not any(several.match(_norm(r["Kernel_Name"])) for r in rows[a + 1:b + 1])][2:]
