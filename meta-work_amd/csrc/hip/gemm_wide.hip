@@ -442,7 +442,7 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const WideArgs a
                     if (tid < kToks) {
                         const int t = min(tg * kToks + tid, a.T - 1);
                         double sum = 0;
-                        for (int b = 0; b < nb; b++) sum += a.ss[(int64_t)b * a.T + t];
+                        for (int b = 0; b < nb; b++) sum += a.ss[(int64_t)b * a.ss_n + t];
                         tsc[tid] = 1.0f / sqrtf((float)(sum / a.K) + a.eps);
                     }
                     __syncthreads();
@@ -694,7 +694,7 @@ __global__ __launch_bounds__(512, 2) void gemm_skinny_kernel(const WideArgs a) {
         if (tid < 16 * NT) {
             const int t = min(tid, a.T - 1);
             double sum = 0;
-            for (int b = 0; b < nb; b++) sum += a.ss[(int64_t)b * a.T + t];
+            for (int b = 0; b < nb; b++) sum += a.ss[(int64_t)b * a.ss_n + t];
             tsc[tid] = 1.0f / sqrtf((float)(sum / a.K) + a.eps);
         }
     }
@@ -874,9 +874,10 @@ int launch_s2(const WideArgs &a, int grid, hipStream_t st) {
 // Q6_K two in three (27.8; three in four 31.0).
 struct SkPlan {
     int rt, ks;
+    double cost;
 };
 SkPlan skinny_plan(bool q6, int tiles, int nb, int nt) {
-    SkPlan best{1, 1};
+    SkPlan best{1, 1, 0.0};
     double lo = 1e30;
     for (int rt = 1; rt <= (q6 ? 3 : 5); rt++)
         for (int ks = 1; ks <= 16 && ks <= nb; ks++) {
@@ -884,9 +885,24 @@ SkPlan skinny_plan(bool q6, int tiles, int nb, int nt) {
             if (ks > 1 && rounds > 1) break;
             const int cw = ((4 * nb + ks - 1) / ks + 7) / 8;
             const double c = rounds * ((rt * (0.5 + 0.5 * nt) + 1.5) * cw + 4.0) + (ks > 1 ? 6.0 + 0.5 * rt * ks : 0.0);
-            if (c < lo) lo = c, best = SkPlan{rt, ks};
+            if (c < lo) lo = c, best = SkPlan{rt, ks, c};
         }
     return best;
+}
+
+// Whether T > 64 tokens go as slices of 64 on the narrow kernel: the wide one's
+// tiles are few for small matrices, each shared by many work-groups whose
+// partial sums one of them adds. Estimates in us, fitted to both kernels (wide /
+// slices): 2560 x 4096 Q4_K at 128 tokens 46 / 27, at 192 50 / 42, at 256 51 /
+// 57; 2560 x 9216 Q6_K at 128 84 / 55, at 192 77 / 82; 7168 x 1024 Q4_K at 128
+// 23 / 16, at 256 27 / 33; 18432 x 2560 Q4_K at 128 45 / 55.
+bool in_slices(const WideArgs &a, int rows16) {
+    const bool q6 = a.type == XJ_Q6_K;
+    const double slice = 2.5 + (q6 ? 0.45 : 0.38) * skinny_plan(q6, rows16, a.nb, 4).cost;
+    const int64_t tiles = (int64_t)((rows16 + 15) / 16) * ((a.T + kToks - 1) / kToks), P = tiles * a.nb;
+    const int64_t units = (P + wide_cus() - 1) / wide_cus(), share = (a.nb + units - 1) / units;
+    const double wide = 10.0 + (q6 ? 10.0 : 9.0) * units + 1.8 * share;
+    return (a.T + kSkinnyT - 1) / kSkinnyT * slice < wide;
 }
 
 }  // namespace
@@ -919,6 +935,7 @@ int wide_prep_launch(const WidePrep &in, hipStream_t st) {
 
 int gemm_wide_launch(const WideArgs &in, int64_t part_floats, int n_cnt, hipStream_t st) {
     WideArgs a = in;
+    if (!a.ss_n) a.ss_n = a.T;
     if ((a.type != XJ_Q4_K && a.type != XJ_Q6_K) || a.K < 256 || a.K % 256 || a.T < 1 || a.nseg < 1 || a.nseg > kGemmMaxSeg ||
         !a.wq || !a.part || !a.cnt || ((uintptr_t)a.wq & 15))
         return -1;
@@ -930,6 +947,19 @@ int gemm_wide_launch(const WideArgs &in, int64_t part_floats, int n_cnt, hipStre
     }
     for (int i = a.nseg + 1; i <= kGemmMaxSeg; i++) a.rt0[i] = a.rt0[a.nseg];
     a.nb = a.K / 256;
+    int rows16 = 0;
+    for (int i = 0; i < a.nseg; i++) rows16 += (a.seg[i].N + 15) / 16;
+    if (a.T > kSkinnyT && in_slices(a, rows16)) {
+        for (int t0 = 0; t0 < a.T; t0 += kSkinnyT) {
+            WideArgs b = a;
+            b.T = std::min(kSkinnyT, a.T - t0);
+            b.wq += (int64_t)(t0 / 32) * a.nb * kWideRec;
+            if (b.ss) b.ss += t0;
+            for (int i = 0; i < a.nseg; i++) b.seg[i].y += (int64_t)t0 * a.seg[i].ys;
+            if (gemm_wide_launch(b, part_floats, n_cnt, st)) return -1;
+        }
+        return 0;
+    }
     if (a.T <= kSkinnyT) {
         const bool q6 = a.type == XJ_Q6_K;
         const int nt = a.T <= 48 ? 3 : 4;

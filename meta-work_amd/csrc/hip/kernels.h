@@ -191,6 +191,7 @@ struct WideArgs {
     int32_t nseg;
     GemmSeg seg[kGemmMaxSeg];
     const double *ss; float eps;    // optional: y[t][r] = sum * rms scale of token t (from the sums of x^2)
+    int32_t ss_n;                   // tokens per block in ss (0: T)
     float *part;                    // wide_part_floats(T) floats
     int32_t *cnt;                   // wide_counters(rows, T) ints, zero before the first launch, left zero
     // set by gemm_wide_launch

@@ -453,11 +453,11 @@ def test_short_chunk_on_the_gemm(tiny, T):
 
 @pytest.mark.parametrize("T", [65, 96, 129, 200, 256])
 def test_wide_chunk_equals_chunks_of_64(tiny, T):
-    """A chunk beyond 64 tokens takes the wide GEMM (256 x 128 tiles over
-    every segment, token tiles of 32: 65 = two and a row, 129 = a second
-    token group of one token) and attention in slices; its hidden rows are
-    those of the same tokens in chunks of 64 on the other GEMM, and the state
-    it leaves serves a decode step. Both round only in fp32 sums: 1e-6 of a
+    """A chunk beyond 64 tokens takes the narrow GEMM in slices of 64 (65: a
+    slice of one token) or, for the tiny model's matrices from 193 tokens on,
+    the wide one (256 x 128 tiles over every segment; 200 and 256: a ragged
+    and a whole second token group); its hidden rows are those of the same
+    tokens in chunks of 64, and the state it leaves serves a decode step. Both round only in fp32 sums: 1e-6 of a
     product, 6e-6 after four layers."""
     m, L = tiny, tiny.hp.n_layer
     toks = prompt_ids(m, T + 1, 300 + T)
