@@ -471,6 +471,48 @@ __device__ __forceinline__ void split2(float x, _Float16 &hi, _Float16 &lo) {
     lo = (_Float16)(x - (float)hi);   // x - hi is exact in fp32
 }
 
+// One query row (token t, head h of kv head g) over the positions [k0, ke) by a
+// wavefront, a lane D / 64 dims, in fp32 and without a masked term; the split's
+// partials or the output row as attn_chunk_kernel leaves them.
+template <int D>
+__device__ __forceinline__ void chunk_row(const AttnArgs &a, int t, int h, int g, int sp, int k0, int ke) {
+    constexpr int NE = D / 64;
+    const int l = threadIdx.x & 63, nk = a.Hkv * D, d0 = g * D + NE * l;
+    float q[NE], o[NE];
+#pragma unroll
+    for (int e = 0; e < NE; e++) q[e] = a.qr[((int64_t)t * a.H + h) * D + NE * l + e], o[e] = 0.f;
+    auto score = [&](int j) {
+        float s = 0.f;
+#pragma unroll
+        for (int e = 0; e < NE; e++) s = fmaf(q[e], xjd::f16_to_f32(a.kc[(int64_t)j * nk + d0 + e]), s);
+        s = xjd::row16_sum(s);
+        s += __shfl_xor(s, 16, 64);
+        s += __shfl_xor(s, 32, 64);
+        return s * a.scale;
+    };
+    float m = -INFINITY, L = 0.f;
+#pragma unroll 4
+    for (int j = k0; j < ke; j++) m = fmaxf(m, score(j));
+#pragma unroll 4
+    for (int j = k0; j < ke; j++) {
+        const float p = expf(score(j) - m);
+        L += p;
+#pragma unroll
+        for (int e = 0; e < NE; e++) o[e] = fmaf(p, xjd::f16_to_f32(a.vc[(int64_t)j * nk + d0 + e]), o[e]);
+    }
+    if (a.n_chunk_sp > 1) {
+        float *part = a.scores + (((int64_t)t * a.H + h) * a.n_chunk_sp + sp) * (D + 4);
+#pragma unroll
+        for (int e = 0; e < NE; e++) part[4 + NE * l + e] = o[e];
+        if (l == 0) part[0] = m, part[1] = L;
+    } else {
+        const int64_t row = (int64_t)t * a.H * D + (int64_t)h * D + NE * l;
+        const float *gp = a.qg + (int64_t)t * a.qg_s + (int64_t)h * 2 * D + D + NE * l;
+#pragma unroll
+        for (int e = 0; e < NE; e++) a.out[row + e] = o[e] * (1.0f / L) * xjd::sigm(gp[e]);
+    }
+}
+
 template <int D, int G>
 __global__ __launch_bounds__(256, 1) void attn_chunk_kernel(const AttnArgs a) {
     constexpr int CH = D / 8;                 // 16-byte pieces per key
@@ -618,8 +660,23 @@ __global__ __launch_bounds__(256, 1) void attn_chunk_kernel(const AttnArgs a) {
             }
         }
     }
-    if (t >= a.T) return;
     constexpr float kP = 1.f / 16384.f;
+    // On the matrix cores a masked key's value is multiplied by the probability 0, and an infinite or NaN value
+    // of a later token (0 x inf = NaN) or the low plane of an infinite one (inf - inf) would reach this row. A
+    // row with a sum that is not finite is formed again from its own keys only (chunk_row); none with finite inputs
+    // (the check costs nothing measurable: a 4B 1024-token prefill 26.1 ms before and after).
+    float fin = 0.f;
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) fin = fmaf(o[d][r], 0.f, fin);   // NaN if any is not finite
+    const uint64_t lanes = __ballot(fin != fin || !(lsum < INFINITY));
+    const uint32_t again = (uint32_t)(lanes | lanes >> 16 | lanes >> 32 | lanes >> 48) & 0xFFFFu;   // rows of the wavefront
+    for (int rr = 0; again >> rr; rr++) {   // uniform
+        const int t2 = tb + (16 * w + rr) / G, h2 = g * G + (16 * w + rr) % G;
+        if ((again >> rr & 1) && t2 < a.T) chunk_row<D>(a, t2, h2, g, sp, k0, min(k1, npast + t2 + 1));
+    }
+    if (t >= a.T || (again >> li & 1)) return;
     if (a.n_chunk_sp > 1) {   // register r of o[d]: dim 16 d + 4 kq + r
         float *part = a.scores + (((int64_t)t * a.H + h) * a.n_chunk_sp + sp) * (D + 4);
 #pragma unroll

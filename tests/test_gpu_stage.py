@@ -547,3 +547,29 @@ def test_chunk_conv_equals_single_steps(model_dir, conv_k, s_k, T):
     assert rel_l2(ya, yb) < 5e-5
     for s in (a, b):
         s.destroy()
+
+
+@pytest.mark.parametrize("H,Hkv,D", [(8, 1, 64), (4, 1, 256)])
+@pytest.mark.parametrize("n_past,T,bad", [(0, 16, 5), (63, 17, 10), (200, 33, 20), (0, 130, 100)])
+def test_nan_token_leaves_earlier_rows_alone(model_dir, H, Hkv, D, n_past, T, bad):
+    """A token whose row is NaN, in the middle of a chunk on the matrix cores
+    (one split and several): the rows before it see neither its key nor its
+    value, so they are those of the same chunk with a finite row there (the
+    bound of two orders of the same fp32 sums, as against single steps); every
+    row from it on is NaN."""
+    from conftest import synth_model
+    cfg = xp.TINY.with_(n_layer=4, n_head=H, n_head_kv=Hkv, head_dim=D)
+    m = xp.Model(synth_model(model_dir, cfg, "tiny_h%d_%d_%d" % (H, Hkv, D)))
+    s = xp.HipStage(m, 3, 4, 288, 144, False)   # the attention layer alone
+    rows = np.random.default_rng(T + n_past).standard_normal((n_past + T, cfg.n_embd)).astype(np.float32)
+    if n_past:
+        for i in range(0, n_past, 100):
+            s.forward(rows[i:min(i + 100, n_past)].copy())
+    want = s.forward(rows[n_past:].copy())
+    s.rollback(n_past)
+    x = rows[n_past:].copy()
+    x[bad] = np.nan
+    got = s.forward(x)
+    assert rel_l2(got[:bad], want[:bad]) < 5e-5
+    assert np.isnan(got[bad:]).all()
+    s.destroy()
