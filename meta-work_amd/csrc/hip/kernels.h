@@ -289,10 +289,11 @@ size_t delta_chunked_work_bytes(int H, int S, int T, int chunk);
 // rollbacks to a checkpoint). Entries past kCopyMax take further launches.
 constexpr int kCopyMax = 48;
 struct CopyList {
-    const float *src[kCopyMax];   // null: dst is set to zero
+    const float *src[kCopyMax];
     float *dst[kCopyMax];
     int64_t n[kCopyMax];   // floats
     int32_t cnt;
+    bool zero;             // every dst is set to zero, src not used
 };
 int copy_list_launch(const CopyList &c, hipStream_t st);
 

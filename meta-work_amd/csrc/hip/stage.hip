@@ -758,10 +758,11 @@ int hip_logits(xj_stage *s, const float *x, int T, float *logits, char *err, siz
 
 // The conv and recurrent states of every DeltaNet layer copied in one launch
 // (per-layer copies cost a launch each): pick(L, conv_src, conv_dst,
-// ssm_src, ssm_dst) names each layer's ends.
+// ssm_src, ssm_dst) names each layer's ends. zero: the destinations are cleared.
 template <class F>
-static int states_copy(HStage *S, hipStream_t st, F pick) {
+static int states_copy(HStage *S, hipStream_t st, F pick, bool zero = false) {
     CopyList c{};
+    c.zero = zero;
     for (auto &L : S->L) {
         if (!L.rec) continue;
         const float *cs = nullptr, *ss = nullptr;
@@ -814,7 +815,7 @@ void hip_reset(xj_stage *s) {
     hipError_t e = states_copy(S, S->st, [&](HLayer &L, const float *&, float *&cd, const float *&, float *&sd) {
                        cd = L.conv;
                        sd = L.ssm;
-                   }) ? hipErrorLaunchFailure : hipSuccess;
+                   }, true) ? hipErrorLaunchFailure : hipSuccess;
     const hipError_t e2 = hipStreamSynchronize(S->st);
     if (e == hipSuccess) e = e2;
     if (e == hipSuccess) e = hipGetLastError();
