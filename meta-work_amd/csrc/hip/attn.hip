@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void kv_store_kernel(const AttnArgs a) {
     __shared__ float buf[kMaxGroup + 1][D];
     __shared__ float2 cs[D / 2];
     __shared__ double red[4][kMaxGroup + 1];
-    const int pos = *a.npast + a.t0 + t, nk = a.Hkv * D, w = tid >> 6;
+    const int pos = *a.npast + t, nk = a.Hkv * D, w = tid >> 6;
     const bool in = tid < D;
     float v[kMaxGroup + 1];
 #pragma unroll
@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void attn_part_kernel(const AttnArgs a) {
     float v[G + 1], vv = 0.f;
     float2 csv = {0.f, 0.f};
     float qnw = 0.f, knw = 0.f;
-    const int npast = *a.npast + a.t0;
+    const int npast = *a.npast;
     if constexpr (F) {
         const bool in = tid < D;
         const int dc = in ? tid : D - 1;
@@ -371,7 +371,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const AttnArgs a) {
 #pragma unroll
     for (int s = 0; s < 64; s++) pv[s] = part[(int64_t)(s < a.n_split ? s : a.n_split - 1) * (D + 2) + 2 + dc];
     const float gx = a.qg[(int64_t)t * a.qg_s + (int64_t)h * 2 * D + D + dc];   // the output gate
-    const int pos = *a.npast + a.t0 + t, ns = pos / kSplitP + 1;
+    const int pos = *a.npast + t, ns = pos / kSplitP + 1;
     __shared__ float w[64];
     __shared__ float inv_l;
     if (tid < 64) {
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(256, 1) void attn_chunk_kernel(const AttnArgs a) {
     const int tid = threadIdx.x, w = tid >> 6, l = tid & 63, li = l & 15, kq = l >> 4;
     const int g = blockIdx.y, sp = blockIdx.z, nk = a.Hkv * D;
     const int tb = ((int)gridDim.x - 1 - (int)blockIdx.x) * TQ;   // the longest rows first
-    const int npast = *a.npast + a.t0;
+    const int npast = *a.npast;
     const int last = npast + min(tb + TQ, a.T) - 1;               // the work-group's last position
     const int k0 = sp * a.sp, k1 = min(k0 + a.sp, last + 1);
     if (k0 > last) return;
@@ -702,7 +702,7 @@ __global__ __launch_bounds__(D) void attn_chunk_merge_kernel(const AttnArgs a) {
     const int h = blockIdx.x, t = blockIdx.y, d = threadIdx.x;
     const float *part = a.scores + ((int64_t)t * a.H + h) * a.n_chunk_sp * (D + 4);
     const float gx = a.qg[(int64_t)t * a.qg_s + (int64_t)h * 2 * D + D + d];
-    const int ns = (*a.npast + a.t0 + t) / a.sp + 1;
+    const int ns = (*a.npast + t) / a.sp + 1;
     float M = -INFINITY;
     for (int s = 0; s < ns; s++) M = fmaxf(M, part[s * (D + 4)]);
     float o = 0.f, L = 0.f;
@@ -786,7 +786,7 @@ static bool attn_args_ok(const AttnArgs &a) {
            a.n_split == attn_splits(a.n_ctx) && a.qr;
 }
 
-// T tokens at positions n_past .. (n_past = *a.npast + a.t0, known to the
+// T tokens at positions n_past .. (n_past = *a.npast, known to the
 // caller) on the matrix cores; scores holds score_floats floats; xq is not written.
 int attn_chunk_launch(const AttnArgs &a, int n_past, int64_t score_floats, hipStream_t st) {
     if (!attn_args_ok(a) || a.T < 1 || n_past < 0 || n_past + a.T > a.n_ctx || !a.scores ||

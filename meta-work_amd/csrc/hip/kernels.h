@@ -227,7 +227,6 @@ struct AttnArgs {
     int32_t T, H, Hkv, D, n_rot, n_ctx, n_split;
     float eps, scale;
     uint8_t *xq;                         // optional: prepared activations of out (no prologue)
-    int32_t t0;                          // token 0 sits at position *npast + t0
     int32_t sp, n_chunk_sp;              // set by attn_chunk_launch: positions per split, splits
 };
 int attn_launch(const AttnArgs &a, hipStream_t st);

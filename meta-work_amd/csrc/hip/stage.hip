@@ -481,7 +481,7 @@ struct Gemv {
 
 // --------------------------------------------------------------- layers --
 
-constexpr int kAttnT = 64;   // tokens per attention launch of a long piece
+constexpr int kScoreT = 64;   // tokens whose attention partials the scratch holds
 
 // Layer il on T tokens of x. The GEMVs that read the residual stream build
 // their RMSNorm activations inside their own work-groups; every other
@@ -576,22 +576,14 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
         at.eps = hp.eps; at.scale = 1.0f / sqrtf((float)D);
         Gemv q = gemv(S->xq_att);
         q.seg(L.wo, x, E, EPI_ADD);
-        // chunks on the matrix cores leave wo's input to its own prep launch; shorter ones, and those kept on
-        // the GEMV's arithmetic, take the decode kernels, in slices of the split partials' scratch
+        // chunks on the matrix cores leave wo's input to its own prep launch; shorter ones take the decode kernels
         if (!pf && T >= kChunkMinT) {
             if (attn_chunk_launch(at, S->s.n_past, S->score_floats, st)) return -1;
             q.a.x = S->o; q.a.xs = Hq * D; q.a.pro = PRO_NONE;
         } else {
+            at.xq = S->xq_att;
+            if (!pf && attn_launch(at, st)) return -1;
             q.prepared = true;
-            for (int t0 = 0; !pf && t0 < T; t0 += kAttnT) {
-                AttnArgs b = at;
-                b.t0 = t0;
-                b.T = T - t0 < kAttnT ? T - t0 : kAttnT;
-                b.qg += (int64_t)t0 * at.qg_s; b.kn += (int64_t)t0 * at.kn_s; b.vn += (int64_t)t0 * at.vn_s;
-                b.out += (int64_t)t0 * Hq * D;
-                b.xq = S->xq_att + (int64_t)t0 * xq_off(Hq * D).stride;
-                if (attn_launch(b, st)) return -1;
-            }
         }
         if (q.run(T, st)) return -1;
     }
@@ -852,7 +844,7 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
     S->g = dalloc<float>(S, mb * sf, err, errlen);
     S->u = dalloc<float>(S, mb * sf, err, errlen);
     S->qr = dalloc<float>(S, mb * hp.n_head * (size_t)hp.head_dim, err, errlen);
-    S->score_floats = (int64_t)(mb < kAttnT ? mb : kAttnT) * hp.n_head * attn_splits(n_ctx) * (hp.head_dim + 2);
+    S->score_floats = (int64_t)(mb < kScoreT ? mb : kScoreT) * hp.n_head * attn_splits(n_ctx) * (hp.head_dim + 2);
     S->scores = dalloc<float>(S, (size_t)S->score_floats, err, errlen);
     S->npast = dalloc<int32_t>(S, 1, err, errlen);
     // prefill on the matrix cores
@@ -974,7 +966,7 @@ extern "C" uint64_t xj_hip_stage_state_bytes(const xj_model *m, int l0, int l1, 
             b += 2ull * 2 * n_ctx * hp.n_head_kv * hp.head_dim;
     }
     b += 10ull * 4 * max_batch * scratch_floats(hp) +
-         4ull * (max_batch < kAttnT ? max_batch : kAttnT) * hp.n_head * ((n_ctx + 63) / 64) * (hp.head_dim + 2);
+         4ull * (max_batch < kScoreT ? max_batch : kScoreT) * hp.n_head * ((n_ctx + 63) / 64) * (hp.head_dim + 2);
     // prefill on the matrix cores: RMSNorm scales, K-split partials and counters, chunked-rule work
     const int64_t grows = 2 * (int64_t)scratch_floats(hp) + 2 * (int64_t)hp.h_v;
     b += 4ull * max_batch + 4ull * gemm_part_floats(grows, max_batch < gemm_max_tokens() ? max_batch : gemm_max_tokens()) +
