@@ -51,10 +51,11 @@ struct WideBuf {
 // Chunks of at least kGemmMinT tokens take the matrix-core GEMM, of at least
 // kChunkMinT also the chunked delta rule and the matrix-core attention. Up to
 // ten tokens (two GEMV launches) a chunk keeps the single token's arithmetic
-// bit for bit, so that what a verification or its rollback leaves equals the
-// tokens fed alone; from eleven on that would take three launches, 52 us
-// against the GEMM's 21 us for 18432 x 2560 Q4_K at twelve. The DeltaNet step
-// kernel costs 2 us a token, the chunked rule 35 us with its preparation.
+// bit for bit; from eleven on that would take three launches, 52 us against the
+// GEMM's 21 us for 18432 x 2560 Q4_K at twelve. A chunk with checkpoints (a
+// verification) keeps it below kChunkMinT whatever it costs: its rows, and what
+// a rollback leaves, equal the tokens fed alone. The DeltaNet step kernel costs
+// 2 us a token, the chunked rule 35 us with its preparation.
 constexpr int kGemmMinT = 11, kChunkMinT = 16;
 
 struct HLayer {
@@ -286,8 +287,9 @@ struct Gemv {
     bool hq_ready = false;
     bool hq_out = false;   // set by a GEMM run whose SwiGLU prep built the next input's hq
     bool raw_conv = false; // a GEMM run leaves the conv segment's projections as they are
+    int min_t = kGemmMinT; // tokens from which the GEMM is taken (with checkpoints kChunkMinT)
     const WideBuf *wide = nullptr;
-    // Chunks of at least kGemmMinT tokens take the matrix-core GEMM
+    // Chunks of at least min_t tokens take the matrix-core GEMM
     // (gemm.hip): the prep launch builds the T tokens' activations once, the
     // RMSNorm scale is applied per token after the dot products (as the GEMV
     // applies it), the conv + SiLU runs as its own launch and the SwiGLU tail
@@ -295,7 +297,7 @@ struct Gemv {
     // rows) and every other case keep the GEMV.
     bool gemm_ok(int T) const {
         static const bool on = env_int("XJ_PREFILL_GEMM", 1) != 0;
-        if (!on || T < kGemmMinT || prof || !tsc || !part || !cnt || !a.xq || !hq) return false;
+        if (!on || T < min_t || prof || !tsc || !part || !cnt || !a.xq || !hq) return false;
         if (a.pro != PRO_NONE && a.pro != PRO_RMSU && a.pro != PRO_SWIGLU && a.pro != PRO_GATED_RMS) return false;
         if (a.post.mode != POST_NONE && a.post.mode != POST_SWIGLU) return false;
         if (a.K % 256) return false;
@@ -492,7 +494,11 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
     HLayer &L = S->L[il - S->s.l0];
     const int E = hp.n_embd, FF = hp.n_ff;
     // every GEMV of the layer with the stage's prefill buffers
-    auto gemv = [&](uint8_t *xq) { return Gemv(xq, pf, S->tsc, S->gpart, S->gpart_floats, S->gcnt, S->n_gcnt, S->hq, &S->wide); };
+    auto gemv = [&](uint8_t *xq) {
+        Gemv g(xq, pf, S->tsc, S->gpart, S->gpart_floats, S->gcnt, S->n_gcnt, S->hq, &S->wide);
+        if (keep_n > 0) g.min_t = kChunkMinT;
+        return g;
+    };
     auto rms_in = [&](Gemv &g, const float *w) {
         g.a.x = x; g.a.xs = E; g.a.pro = PRO_RMSU; g.a.pro_w = w; g.a.eps = hp.eps;
     };
