@@ -58,6 +58,8 @@ struct WideBuf {
 // 2 us a token, the chunked rule 35 us with its preparation.
 constexpr int kGemmMinT = 11, kChunkMinT = 16;
 
+constexpr size_t kPieceScoreT = 64;   // tokens whose attention partials the pieces' scratch holds
+
 struct HLayer {
     bool rec = false;
     const float *attn_norm = nullptr, *post_norm = nullptr;
@@ -107,6 +109,7 @@ struct HStage {
     int32_t *gcnt = nullptr;   // the GEMM's arrival counters (zero between launches)
     int32_t n_gcnt = 0;
     WideBuf wide;              // buffers of the wide GEMM (max_batch > 64)
+    bool pieces = false;       // scratch for prompt pieces (twin_new)
     float2 *rope = nullptr;
     float *h_x = nullptr;            // pinned staging [max_batch][n_embd]
     int32_t *h_i = nullptr;          // pinned scalar
@@ -124,6 +127,13 @@ thread_local char g_lasterr[512];
 int env_int(const char *k, int def) {
     const char *v = getenv(k);
     return v ? atoi(v) : def;
+}
+
+// Chunks on the matrix cores (their GEMMs, attention and prompt pieces); the
+// chunked delta rule has a switch of its own.
+bool prefill_gemm() {
+    static const bool on = env_int("XJ_PREFILL_GEMM", 1) != 0;
+    return on;
 }
 
 HStage *H(xj_stage *s) { return reinterpret_cast<HStage *>(s); }
@@ -296,8 +306,7 @@ struct Gemv {
     // as the down projection's prep. Segments the GEMM does not take (float
     // rows) and every other case keep the GEMV.
     bool gemm_ok(int T) const {
-        static const bool on = env_int("XJ_PREFILL_GEMM", 1) != 0;
-        if (!on || T < min_t || prof || !tsc || !part || !cnt || !a.xq || !hq) return false;
+        if (!prefill_gemm() || T < min_t || prof || !tsc || !part || !cnt || !a.xq || !hq) return false;
         if (a.pro != PRO_NONE && a.pro != PRO_RMSU && a.pro != PRO_SWIGLU && a.pro != PRO_GATED_RMS) return false;
         if (a.post.mode != POST_NONE && a.post.mode != POST_SWIGLU) return false;
         if (a.K % 256) return false;
@@ -483,8 +492,6 @@ struct Gemv {
 
 // --------------------------------------------------------------- layers --
 
-constexpr int kScoreT = 64;   // tokens whose attention partials the scratch holds
-
 // Layer il on T tokens of x. The GEMVs that read the residual stream build
 // their RMSNorm activations inside their own work-groups; every other
 // prologue is produced by the kernel before its GEMV: the down input by
@@ -574,6 +581,9 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
             p.seg(L.wq, S->qkv, nq, EPI_STORE).seg(L.wk, S->kb, nk, EPI_STORE).seg(L.wv, S->vb, nk, EPI_STORE);
             at.qg = S->qkv; at.qg_s = nq; at.kn = S->kb; at.kn_s = nk; at.vn = S->vb; at.vn_s = nk;
         }
+        // a chunk on the matrix cores; with checkpoints only if its projections are, so that one kept on the
+        // GEMV's arithmetic keeps the single token's bits
+        const bool chunk = !pf && prefill_gemm() && T >= kChunkMinT && (keep_n == 0 || p.gemm_ok(T));
         if (p.run(T, st)) return -1;
         at.kc = L.kc; at.vc = L.vc; at.qnorm_w = L.q_norm; at.knorm_w = L.k_norm; at.rope = S->rope;
         at.npast = S->npast; at.qr = S->qr; at.scores = S->scores; at.out = S->o;
@@ -582,8 +592,8 @@ int enqueue_layer(HStage *S, int il, float *x, int T, int keep_n, int32_t *inc, 
         at.eps = hp.eps; at.scale = 1.0f / sqrtf((float)D);
         Gemv q = gemv(S->xq_att);
         q.seg(L.wo, x, E, EPI_ADD);
-        // chunks on the matrix cores leave wo's input to its own prep launch; shorter ones take the decode kernels
-        if (!pf && T >= kChunkMinT) {
+        // chunks on the matrix cores leave wo's input to its own prep launch; others take the decode kernels
+        if (chunk) {
             if (attn_chunk_launch(at, S->s.n_past, S->score_floats, st)) return -1;
             q.a.x = S->o; q.a.xs = Hq * D; q.a.pro = PRO_NONE;
         } else {
@@ -850,7 +860,10 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
     S->g = dalloc<float>(S, mb * sf, err, errlen);
     S->u = dalloc<float>(S, mb * sf, err, errlen);
     S->qr = dalloc<float>(S, mb * hp.n_head * (size_t)hp.head_dim, err, errlen);
-    S->score_floats = (int64_t)(mb < kScoreT ? mb : kScoreT) * hp.n_head * attn_splits(n_ctx) * (hp.head_dim + 2);
+    // attention partials: of every token for the decode kernels; pieces (beyond max_batch, on the matrix cores)
+    // need them only where few query rows are split
+    const size_t score_t = S->pieces && mb > kPieceScoreT ? kPieceScoreT : mb;
+    S->score_floats = (int64_t)score_t * hp.n_head * attn_splits(n_ctx) * (hp.head_dim + 2);
     S->scores = dalloc<float>(S, (size_t)S->score_floats, err, errlen);
     S->npast = dalloc<int32_t>(S, 1, err, errlen);
     // prefill on the matrix cores
@@ -909,6 +922,7 @@ static HStage *twin_new(HStage *S, int max_batch, char *err, size_t errlen) {
     HStage *T = new HStage();
     T->s = S->s;
     T->s.max_batch = max_batch;
+    T->pieces = true;
     T->st = S->st;
     T->rope = S->rope;
     T->conv_n = S->conv_n; T->ssm_n = S->ssm_n;
@@ -972,7 +986,7 @@ extern "C" uint64_t xj_hip_stage_state_bytes(const xj_model *m, int l0, int l1, 
             b += 2ull * 2 * n_ctx * hp.n_head_kv * hp.head_dim;
     }
     b += 10ull * 4 * max_batch * scratch_floats(hp) +
-         4ull * (max_batch < kScoreT ? max_batch : kScoreT) * hp.n_head * ((n_ctx + 63) / 64) * (hp.head_dim + 2);
+         4ull * max_batch * hp.n_head * ((n_ctx + 63) / 64) * (hp.head_dim + 2);
     // prefill on the matrix cores: RMSNorm scales, K-split partials and counters, chunked-rule work
     const int64_t grows = 2 * (int64_t)scratch_floats(hp) + 2 * (int64_t)hp.h_v;
     b += 4ull * max_batch + 4ull * gemm_part_floats(grows, max_batch < gemm_max_tokens() ? max_batch : gemm_max_tokens()) +
@@ -1246,8 +1260,7 @@ struct xjh_chain {
 // Every stage's scratch for prompt pieces, created once; false: none (max_batch
 // too large to need it, or no memory: prompts then run in chunks of max_batch).
 static bool chain_twins(xjh_chain *c) {
-    static const bool on = env_int("XJ_PREFILL_GEMM", 1) != 0;
-    if (!on || c->mb > kPieceT / 2 || c->piece < 0) return false;
+    if (!prefill_gemm() || c->mb > kPieceT / 2 || c->piece < 0) return false;
     if (c->piece > 0) return true;
     char err[256];
     const int n_ctx = (c->st[0]->s.n_ctx + 127) / 128 * 128;

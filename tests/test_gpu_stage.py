@@ -5,6 +5,11 @@ Mirrors the reference's own GPU-vs-CPU check (src/xiaoju-pipe/tools/xjpipe-check
 prefill 12 tokens then 3 single tokens, head top-1, keep/rollback equal to
 never having computed the rolled-back tokens; plus greedy token identity.
 """
+import os
+import subprocess
+import sys
+import textwrap
+
 import numpy as np
 import pytest
 
@@ -22,6 +27,14 @@ def tiny(tiny_path):
 
 def embed(m, toks):
     return np.stack([orc.embed(m.ptr, int(t)) for t in toks]).astype(np.float32)
+
+
+def in_child(code, **env):
+    """Runs `code` in a python of its own, with switches the library reads once per process."""
+    path = os.pathsep.join(p for p in sys.path if p)
+    r = subprocess.run([sys.executable, "-c", textwrap.dedent(code)], env=dict(os.environ, PYTHONPATH=path, **env),
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
 
 
 def prompt_ids(m, n, seed):
@@ -590,3 +603,25 @@ def test_nan_token_leaves_earlier_rows_alone(model_dir, H, Hkv, D, n_past, T, ba
     assert rel_l2(got[:bad], want[:bad]) < 5e-5
     assert np.isnan(got[bad:]).all()
     s.destroy()
+
+
+def test_chunk_on_the_gemv_keeps_the_steps_bits(tiny_path):
+    """Chunks kept on the GEMV's arithmetic (XJ_PREFILL_GEMM=0, read once per
+    process) take the decode's attention too: 70 rows with checkpoints, and a
+    step after a rollback into them, are those of the rows fed one at a time,
+    bit for bit."""
+    in_child(f"""
+        import numpy as np, xjpipe as xp
+        m = xp.Model({tiny_path!r})
+        rows = np.random.default_rng(5).standard_normal((72, m.hp.n_embd)).astype(np.float32)
+        a, b = (xp.HipStage(m, 0, m.hp.n_layer, 128, 96, False) for _ in range(2))
+        a.set_keep(70)
+        ya = a.forward(rows[:70].copy())
+        yb = np.concatenate([b.forward(rows[i:i + 1].copy()) for i in range(33)])
+        assert np.array_equal(ya[:33].view(np.uint32), yb.view(np.uint32))
+        a.rollback(33)
+        ya, yb = (s.forward(rows[70:71].copy()) for s in (a, b))
+        assert np.array_equal(ya.view(np.uint32), yb.view(np.uint32))
+        for s in (a, b):
+            s.destroy()
+        """, XJ_PREFILL_GEMM="0")
