@@ -69,11 +69,15 @@ const char *xj_hip_tune_note(void);
 
 /* Bytes of HBM a stage holds besides the repacked weights
  * (counterpart of xj_stage_state_bytes, xj_stage.h:57). A chain
- * (xjh_chain_new) over stages of max_batch <= 512 adds a second set of scratch
- * per stage, for prompts beyond max_batch in pieces of up to
- * min(n_ctx, 1024) tokens: when it is built if max_batch >= 16, else on the
- * first such prompt of 16 tokens or more. Without the memory for it, prompts
- * run in chunks of max_batch. */
+ * (xjh_chain_new) over stages of max_batch <= 512 whose matrices are mostly
+ * Q4_K and Q6_K adds a second set of scratch per stage, for prompts beyond
+ * max_batch in pieces of up to min(n_ctx, 1024) tokens: when it is built if
+ * max_batch >= 16, else on the first prompt of 16 tokens or more beyond two
+ * chunks. Other prompts beyond max_batch run in chunks of max_batch, a single
+ * stage's layers in up to XJ_STAGE_SPLIT parts, for which the chain adds up to
+ * XJ_STAGE_SPLIT - 1 further sets of the stage's own scratch: when it is built
+ * if max_batch >= 16 and there are no pieces, else on the first such prompt.
+ * Without the memory for them, chunks run one after the other. */
 uint64_t    xj_hip_stage_state_bytes(const xj_model *m, int l0, int l1, int n_ctx, int max_batch);
 
 /* Copy the whole recurrent state (conv + DeltaNet state of every layer) of a

@@ -915,14 +915,14 @@ static bool alloc_scratch(HStage *S, char *err, size_t errlen) {
     return true;
 }
 
-// A second set of scratch, for pieces of a prompt longer than the stage's
-// max_batch (chain_eval): the stage's weights, layer states and stream, its
-// own position counter.
-static HStage *twin_new(HStage *S, int max_batch, char *err, size_t errlen) {
+// Another set of scratch for a stage (chain_eval): the stage's weights, layer
+// states and stream, its own position counter. For pieces of a prompt of up to
+// max_batch tokens, or for later layers beside the stage's own (pieces false).
+static HStage *twin_new(HStage *S, int max_batch, bool pieces, char *err, size_t errlen) {
     HStage *T = new HStage();
     T->s = S->s;
     T->s.max_batch = max_batch;
-    T->pieces = true;
+    T->pieces = pieces;
     T->st = S->st;
     T->rope = S->rope;
     T->conv_n = S->conv_n; T->ssm_n = S->ssm_n;
@@ -1225,10 +1225,16 @@ extern "C" int xj_hip_stage_restore(xj_stage *s, int slot, int n_past, char *err
 // a weight is decoded once per 128 tokens, and every launch fills the chip.
 // Stages whose max_batch is above half of it run their own chunks.
 constexpr int kPieceT = 1024;
+constexpr int kMaxParts = 4;   // parts of a single stage's layers in a pipelined prefill
 struct xjh_chain {
     std::vector<HStage *> st;
     std::vector<HStage *> twins;   // per stage, scratch for prompt pieces of up to piece tokens (twin_new)
-    int piece = 0;
+    int piece = 0;                 // (-1: no memory for them)
+    // a single stage's layers in parts pipelined over the chunks of a prompt:
+    // scratch and stream of the later ones (a failed allocation: no parts)
+    std::vector<HStage *> parts;
+    std::vector<hipStream_t> part_st;
+    bool parts_failed = false;
     hipStream_t stream = nullptr;
     float *x = nullptr;
     int mb = 0, hist_cap = 0;
@@ -1245,7 +1251,6 @@ struct xjh_chain {
     int32_t *d_prompt = nullptr;
     int prompt_cap = 0;
     std::vector<hipEvent_t> ev_done, ev_taken;
-    hipStream_t half = nullptr;   // a single stage's later layers in a prompt of two short chunks
     // the app's sampler (xjh_chain_set_sampler): temperature, the uniform
     // numbers on the device, how many are drawn; the sampled decode graph
     float temp = 0.f;
@@ -1257,15 +1262,33 @@ struct xjh_chain {
     hipGraph_t graph_s = nullptr;
 };
 
-// Every stage's scratch for prompt pieces, created once; false: none (max_batch
-// too large to need it, or no memory: prompts then run in chunks of max_batch).
+// Whether a stage's prompts gain from pieces: most bytes of its matrices are of
+// the types the GEMM takes. Other matrices stream through the GEMV for every few
+// tokens of a piece as of a chunk, and gain from parts of the layers side by side.
+static bool stage_gemm(const HStage *S) {
+    uint64_t k = 0, all = 0;
+    for (auto &L : S->L)
+        for (const DevW *w : {&L.wq, &L.wk, &L.wv, &L.wqkv, &L.wo, &L.ssm_qkv, &L.ssm_gate, &L.ssm_beta, &L.ssm_alpha, &L.ssm_out,
+                              &L.ffn_gate, &L.ffn_up, &L.ffn_down}) {
+            all += w->bytes;
+            if (w->type == XJ_Q4_K || w->type == XJ_Q6_K) k += w->bytes;
+        }
+    return 2 * k >= all;
+}
+static bool chain_pieces(const xjh_chain *c) {
+    bool ok = prefill_gemm() && c->mb <= kPieceT / 2;
+    for (auto *S : c->st) ok = ok && stage_gemm(S);
+    return ok;
+}
+// Every stage's scratch for prompt pieces, created once; false: none (pieces
+// bring nothing, or no memory: prompts then run in chunks of max_batch).
 static bool chain_twins(xjh_chain *c) {
-    if (!prefill_gemm() || c->mb > kPieceT / 2 || c->piece < 0) return false;
+    if (c->piece < 0 || !chain_pieces(c)) return false;
     if (c->piece > 0) return true;
     char err[256];
     const int n_ctx = (c->st[0]->s.n_ctx + 127) / 128 * 128;
     for (auto *S : c->st) {
-        HStage *T = twin_new(S, n_ctx < kPieceT ? n_ctx : kPieceT, err, sizeof err);
+        HStage *T = twin_new(S, n_ctx < kPieceT ? n_ctx : kPieceT, true, err, sizeof err);
         if (!T) {
             for (HStage *t : c->twins) twin_free(t);
             c->twins.clear();
@@ -1277,6 +1300,34 @@ static bool chain_twins(xjh_chain *c) {
     }
     c->piece = c->twins[0]->s.max_batch;
     return true;
+}
+// Parts of a single stage's layers in a prompt of several chunks
+// (XJ_STAGE_SPLIT, with chunks overlapped on the parts' streams), else 1.
+// Chunks beyond kPieceT / 2 tokens on the GEMM fill the chip one by one.
+static int stage_parts(const xjh_chain *c) {
+    static const bool overlap = env_int("XJ_CHAIN_OVERLAP", 1) != 0;
+    static const int split = env_int("XJ_STAGE_SPLIT", 3);
+    if (c->st.size() != 1 || !overlap || c->parts_failed) return 1;
+    if (c->mb > kPieceT / 2 && prefill_gemm() && stage_gemm(c->st[0])) return 1;
+    const int nl = c->st[0]->s.l1 - c->st[0]->s.l0;
+    return split < 1 ? 1 : split > kMaxParts ? kMaxParts : split > nl ? nl : split;
+}
+// The later parts' scratch (max_batch tokens) and streams, created once; the parts there are.
+static int chain_parts(xjh_chain *c) {
+    char err[256];
+    while ((int)c->parts.size() < stage_parts(c) - 1) {
+        hipStream_t st = nullptr;
+        HStage *T = twin_new(c->st[0], c->mb, false, err, sizeof err);
+        if (!T || hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) {
+            twin_free(T);
+            c->parts_failed = true;
+            (void)hipGetLastError();
+            break;
+        }
+        c->parts.push_back(T);
+        c->part_st.push_back(st);
+    }
+    return (int)c->parts.size() + 1;
 }
 extern "C" void xjh_chain_free(xjh_chain *c) {
     if (!c) return;
@@ -1293,9 +1344,10 @@ extern "C" void xjh_chain_free(xjh_chain *c) {
     for (hipEvent_t e : c->ev_done) if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : c->ev_taken) if (e) (void)hipEventDestroy(e);
     if (c->d_prompt) (void)hipFree(c->d_prompt);
-    if (c->half) (void)hipStreamSynchronize(c->half);
+    for (hipStream_t st : c->part_st) (void)hipStreamSynchronize(st);
     for (HStage *T : c->twins) twin_free(T);
-    if (c->half) (void)hipStreamDestroy(c->half);
+    for (HStage *T : c->parts) twin_free(T);
+    for (hipStream_t st : c->part_st) (void)hipStreamDestroy(st);
     for (int32_t *p : {c->d_tokens, c->d_argmax, c->d_tok, c->d_hist, c->d_step, c->d_rbase, c->d_pick}) if (p) (void)hipFree(p);
     if (c->h_buf) (void)hipHostFree(c->h_buf);
     delete c;
@@ -1333,7 +1385,7 @@ extern "C" xjh_chain *xjh_chain_new(xj_stage **stages, int n, char *err, size_t 
         xjh_chain_free(c);
         return nullptr;
     }
-    const size_t nev = c->st.size() < 2 ? 2 : c->st.size();
+    const size_t nev = c->st.size() < kMaxParts ? kMaxParts : c->st.size();   // a single stage may run in parts
     c->ev_done.assign(nev, nullptr);
     c->ev_taken.assign(nev, nullptr);
     for (size_t i = 0; i < nev; i++)
@@ -1343,9 +1395,9 @@ extern "C" xjh_chain *xjh_chain_new(xj_stage **stages, int n, char *err, size_t 
             xjh_chain_free(c);
             return nullptr;
         }
-    // stages whose chunks take the prefill GEMM get the pieces' scratch now, so
-    // that the first long prompt does not pay for the allocations
-    if (c->mb >= kChunkMinT) (void)chain_twins(c);
+    // stages of ordinary chunks get the scratch of long prompts now, so that
+    // the first one does not pay for the allocations
+    if (c->mb >= kChunkMinT && !chain_twins(c)) (void)chain_parts(c);
     return c;
 }
 
@@ -1357,9 +1409,10 @@ static int chain_sync(xjh_chain *c, char *err, size_t errlen) {
 }
 
 // A prompt longer than max_batch, in pieces: of up to kPieceT tokens on the
-// stages' second scratch (chain_twins), else in chunks of max_batch. The stages are pipelined
+// stages' second scratch (chain_twins), else in chunks of max_batch, a single
+// stage's layers then in parts (chain_parts). Stages and parts are pipelined
 // (pipe/core/xj_net.c:561-604 pipelines a remote worker's half against the
-// host's): each stage runs on its own stream from its own hidden-state buffer,
+// host's): each runs on its own stream from its own hidden-state buffer,
 // so stage i works on piece k + 1 while stage i + 1 works on piece k. Stage
 // i + 1 takes piece k by a device copy once stage i has finished it (event
 // done[i]); stage i overwrites its buffer with piece k + 1 only after that copy
@@ -1386,18 +1439,17 @@ static int chain_eval(xjh_chain *c, const int32_t *tokens, int n, int nlog, int 
     // the pipeline's parts: layers [lo, hi) of a stage S on the scratch of R
     struct Part { HStage *S, *R; int lo, hi; hipStream_t st; };
     std::vector<Part> parts;
-    for (size_t i = 0; i < c->st.size(); i++) {
+    // chunks of max_batch through a single stage: its layers in contiguous parts,
+    // so that a chunk's early layers run beside the one before's later ones (0.8B
+    // on the GEMV, one stream / three parts: 512 tokens in chunks of 64 125 / 89
+    // ms, 128 in chunks of 8 39.0 / 25.0, 16 in chunks of 8 4.9 / 4.2)
+    const int ns = !wide && n > B ? chain_parts(c) : 1, nl = head->s.l1 - head->s.l0;
+    for (int p = 0; ns > 1 && p < ns; p++)
+        parts.push_back(Part{head, p ? c->parts[p - 1] : head, head->s.l0 + nl * p / ns, head->s.l0 + nl * (p + 1) / ns,
+                             p ? c->part_st[p - 1] : head->st});
+    for (size_t i = 0; ns == 1 && i < c->st.size(); i++) {
         HStage *S = c->st[i];
         parts.push_back(Part{S, wide ? c->twins[i] : S, S->s.l0, S->s.l1, overlap ? S->st : c->stream});
-    }
-    // two short chunks through a single stage: its later layers on the second
-    // scratch and a stream of their own, so that the second chunk's launches
-    // run beside the first's (0.8B, 16 tokens, max_batch 8: 5.0 -> 4.5 ms)
-    if (!wide && parts.size() == 1 && n > B && overlap && head->s.l1 - head->s.l0 > 1 && chain_twins(c) && B <= c->piece &&
-        (c->half || hipStreamCreateWithFlags(&c->half, hipStreamNonBlocking) == hipSuccess)) {
-        const int mid = (head->s.l0 + head->s.l1) / 2;
-        parts[0].hi = mid;
-        parts.push_back(Part{head, c->twins[0], mid, head->s.l1, c->half});
     }
     const int np = (int)parts.size();
     auto fail_sync = [&]() {

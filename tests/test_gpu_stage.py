@@ -5,6 +5,7 @@ Mirrors the reference's own GPU-vs-CPU check (src/xiaoju-pipe/tools/xjpipe-check
 prefill 12 tokens then 3 single tokens, head top-1, keep/rollback equal to
 never having computed the rolled-back tokens; plus greedy token identity.
 """
+import ctypes as C
 import os
 import subprocess
 import sys
@@ -625,3 +626,56 @@ def test_chunk_on_the_gemv_keeps_the_steps_bits(tiny_path):
         for s in (a, b):
             s.destroy()
         """, XJ_PREFILL_GEMM="0")
+
+
+def test_short_prompt_takes_little_memory(tiny):
+    """A prompt just beyond a small max_batch must not allocate the scratch of
+    1024-token pieces (over 100 MB for this model, 1 GB for the 4B shape):
+    only further sets of the stage's own scratch, of max_batch tokens."""
+    m, L = tiny, tiny.hp.n_layer
+    path = next(l.split()[-1] for l in open("/proc/self/maps") if "libamdhip64" in l)
+    hip = C.CDLL(path)
+
+    def free():
+        f, t = C.c_size_t(), C.c_size_t()
+        assert hip.hipMemGetInfo(C.byref(f), C.byref(t)) == 0
+        return f.value
+
+    g = xp.HipStage(m, 0, L, 2048, 8, True)
+    ch = xp.Chain([g])
+    before = free()
+    ch.eval(prompt_ids(m, 9, 3))
+    assert before - free() < 32 << 20
+    ch.free()
+    g.destroy()
+
+
+@pytest.mark.parametrize("n,mb,split", [(70, 16, 3), (70, 16, 4), (9, 4, 2), (33, 32, 3)])
+def test_layers_in_parts_equal_chunks_in_turn(tiny_path, n, mb, split):
+    """A prompt that goes in chunks of max_batch through a single stage
+    (XJ_PREFILL_GEMM=0: no pieces) runs its layers in parts on streams of
+    their own, each part's buffer overwritten only once the next has taken it:
+    the logits of the last rows and the tokens decoded after it are those of
+    the same chunks one after the other, bit for bit, twice in a row."""
+    in_child(f"""
+        import numpy as np, xjpipe as xp
+        m = xp.Model({tiny_path!r})
+        L, n, mb = m.hp.n_layer, {n}, {mb}
+        ids = np.random.default_rng(n).integers(0, m.hp.n_vocab, n).astype(np.int32)
+        def tail():
+            return n - (n - 1) // mb * mb
+        a, b = xp.HipStage(m, 0, L, 128, mb, True), xp.HipStage(m, 0, L, 128, mb, True)
+        ca, cb = xp.Chain([a]), xp.Chain([b])
+        for i in range(0, n, mb):
+            am, want = cb.eval(ids[i:i + mb], nlog=tail(), want_logits=True)
+        toks = cb.decode(6).tolist()
+        for _ in range(2):
+            ca.reset()
+            am2, got = ca.eval(ids, nlog=mb, want_logits=True)
+            assert np.array_equal(got[:tail()].view(np.uint32), want.view(np.uint32))
+            assert ca.decode(6).tolist() == toks
+        for o in (ca, cb):
+            o.free()
+        for o in (a, b):
+            o.destroy()
+        """, XJ_PREFILL_GEMM="0", XJ_STAGE_SPLIT=str(split))
