@@ -147,15 +147,28 @@ struct KeptWork {
     size_t cap = 0;
 } g_work;
 
-bool device_alloc(void **p, size_t bytes) {
+// hipMalloc; a failure sets *p to null and leaves no error behind for the next
+// launch's check to find.
+bool plain_alloc(void **p, size_t bytes) {
     if (hipMalloc(p, bytes) == hipSuccess) return true;
+    *p = nullptr;
+    (void)hipGetLastError();
+    return false;
+}
+// Every device allocation of the library but the kept work area itself, whose
+// lock the caller must not hold.
+bool device_alloc(void **p, size_t bytes) {
+    if (plain_alloc(p, bytes)) return true;
     std::unique_lock<std::mutex> lock(g_work.mu, std::try_to_lock);
     if (!lock.owns_lock() || !g_work.p) return false;
     (void)hipFree(g_work.p);
     g_work.p = nullptr;
     g_work.cap = 0;
-    (void)hipGetLastError();
-    return hipMalloc(p, bytes) == hipSuccess;
+    return plain_alloc(p, bytes);
+}
+template <class T>
+bool device_alloc(T **p, size_t bytes) {
+    return device_alloc((void **)p, bytes);
 }
 
 template <class T>
@@ -665,7 +678,7 @@ int ensure_ck(HStage *S, int n, char *err, size_t errlen) {
         if (!L.rec) continue;
         if (L.ck_conv) { (void)hipFree(L.ck_conv); (void)hipFree(L.ck_ssm); }
         L.ck_conv = L.ck_ssm = nullptr;
-        if (hipMalloc(&L.ck_conv, n * S->conv_n * 4) != hipSuccess || hipMalloc(&L.ck_ssm, n * S->ssm_n * 4) != hipSuccess) {
+        if (!device_alloc(&L.ck_conv, n * S->conv_n * 4) || !device_alloc(&L.ck_ssm, n * S->ssm_n * 4)) {
             S->n_ck = 0;
             snprintf(err, errlen, "out of HBM for speculative checkpoints");
             return -1;
@@ -1158,7 +1171,7 @@ static int snapshot_enqueue(HStage *S, int slot, hipStream_t st, char *err, size
     if (slot < 0 || slot >= kSnapSlots) { snprintf(err, errlen, "snapshot slot %d out of range", slot); return -1; }
     for (auto &L : S->L) {
         if (!L.rec || L.snap_conv[slot]) continue;
-        if (hipMalloc(&L.snap_conv[slot], S->conv_n * 4) != hipSuccess || hipMalloc(&L.snap_ssm[slot], S->ssm_n * 4) != hipSuccess) {
+        if (!device_alloc(&L.snap_conv[slot], S->conv_n * 4) || !device_alloc(&L.snap_ssm[slot], S->ssm_n * 4)) {
             snprintf(err, errlen, "out of HBM for snapshots");
             return -1;
         }
@@ -1375,10 +1388,10 @@ extern "C" xjh_chain *xjh_chain_new(xj_stage **stages, int n, char *err, size_t 
     c->mb = S0->s.max_batch;
     for (auto *S : c->st) if (S->s.max_batch < c->mb) c->mb = S->s.max_batch;
     c->hist_cap = 1 << 16;
-    if (hipMalloc(&c->d_tokens, 4 * c->mb) != hipSuccess || hipMalloc(&c->d_argmax, 4 * c->mb) != hipSuccess ||
-        hipMalloc(&c->d_tok, 4) != hipSuccess || hipMalloc(&c->d_hist, 4 * c->hist_cap) != hipSuccess ||
-        hipMalloc(&c->d_step, 4) != hipSuccess || hipMalloc(&c->d_rbase, 4) != hipSuccess ||
-        hipMalloc(&c->d_pick, 4 * c->mb) != hipSuccess || hipMalloc(&c->d_temp, 4) != hipSuccess ||
+    if (!device_alloc(&c->d_tokens, 4 * c->mb) || !device_alloc(&c->d_argmax, 4 * c->mb) ||
+        !device_alloc(&c->d_tok, 4) || !device_alloc(&c->d_hist, 4 * c->hist_cap) ||
+        !device_alloc(&c->d_step, 4) || !device_alloc(&c->d_rbase, 4) ||
+        !device_alloc(&c->d_pick, 4 * c->mb) || !device_alloc(&c->d_temp, 4) ||
         hipHostMalloc((void **)&c->h_buf, 4 * (c->mb + 16), hipHostMallocDefault) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess) {
         snprintf(err, errlen, "chain allocation failed");
@@ -1460,7 +1473,7 @@ static int chain_eval(xjh_chain *c, const int32_t *tokens, int n, int nlog, int 
     if (n > c->prompt_cap) {
         if (c->d_prompt) (void)hipFree(c->d_prompt);
         c->d_prompt = nullptr, c->prompt_cap = 0;
-        if (hipMalloc(&c->d_prompt, 4 * (size_t)n) != hipSuccess) { snprintf(err, errlen, "prompt allocation failed"); return -1; }
+        if (!device_alloc(&c->d_prompt, 4 * (size_t)n)) { snprintf(err, errlen, "prompt allocation failed"); return -1; }
         c->prompt_cap = n;
     }
     // the ids (synchronous copy from the caller's memory) and every part's
@@ -1645,7 +1658,7 @@ extern "C" int xjh_chain_set_sampler(xjh_chain *c, float temperature, const uint
         if (c->d_rnd) (void)hipFree(c->d_rnd);
         c->d_rnd = nullptr;
         c->rnd_cap = 0;
-        if (hipMalloc(&c->d_rnd, 4 * (size_t)n) != hipSuccess) { snprintf(err, errlen, "sampler: hipMalloc failed"); return -1; }
+        if (!device_alloc(&c->d_rnd, 4 * (size_t)n)) { snprintf(err, errlen, "sampler: hipMalloc failed"); return -1; }
         c->rnd_cap = n;
     }
     if ((n > 0 && hipMemcpy(c->d_rnd, rand30, 4 * (size_t)n, hipMemcpyHostToDevice) != hipSuccess) ||
@@ -2194,8 +2207,8 @@ extern "C" int xjh_spec_generate_mtp(xjh_chain *tgt, xj_stage *mtp, int k, const
     if (k > 4) k = 4;
     if (k + 1 > B) k = B - 1;
     if (k > R.S->s.max_batch) k = R.S->s.max_batch;
-    if (hipMalloc(&R.d_ids, 4 * (size_t)R.S->s.max_batch) != hipSuccess || hipMalloc(&R.d_am, 4) != hipSuccess ||
-        hipMalloc(&R.d_hn, sizeof(float) * (size_t)B * E) != hipSuccess) {
+    if (!device_alloc(&R.d_ids, 4 * (size_t)R.S->s.max_batch) || !device_alloc(&R.d_am, 4) ||
+        !device_alloc(&R.d_hn, sizeof(float) * (size_t)B * E)) {
         snprintf(err, errlen, "hipMalloc failed");
         (void)hipFree(R.d_ids); (void)hipFree(R.d_am);
         return -1;
@@ -2398,7 +2411,7 @@ static int gemv_enqueue(uint32_t type, const void *dw, int64_t n_rows, int64_t k
             if (xq_own) (void)hipFree(xq_own);
             xq_own = nullptr;
             xq_cap = 0;
-            if (hipMalloc(&xq_own, need) != hipSuccess) return -1;
+            if (!device_alloc(&xq_own, need)) return -1;
             xq_cap = need;
         }
         xq = xq_own;
@@ -2485,7 +2498,7 @@ static int gemm_enqueue(uint32_t type, const void *dw, int64_t n_rows, int64_t k
         if (need <= cap) return true;
         if (p) (void)hipFree(p);
         p = nullptr, cap = 0;
-        if (hipMalloc(&p, need * sizeof(*p)) != hipSuccess) return false;
+        if (!device_alloc(&p, need * sizeof(*p))) return false;
         cap = need;
         return true;
     };
@@ -2614,7 +2627,7 @@ extern "C" int xjh_rope(float *x, int T, int n_heads, int64_t tok_stride, int64_
     std::vector<float2> cs((size_t)T * half);
     rope_table(pos0, T, n_rot, base, cs.data());
     float2 *d = nullptr;
-    if (hipMalloc(&d, cs.size() * sizeof(float2)) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+    if (!device_alloc(&d, cs.size() * sizeof(float2))) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
     int rc = 0;
     if (hipMemcpy(d, cs.data(), cs.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
         rope_launch(x, d, T, n_heads, tok_stride, head_stride, n_rot, g_stream)) {
@@ -2657,7 +2670,7 @@ extern "C" int xjh_attn_decode(int T, int H, int Hkv, int D, int n_rot, float ro
     const size_t b_rope = (cs.size() * sizeof(float2) + 255) & ~(size_t)255, b_qr = ((size_t)T * H * D * 4 + 255) & ~(size_t)255,
                  b_sc = (size_t)T * H * at.n_split * (D + 2) * 4;
     uint8_t *buf = nullptr;
-    if (hipMalloc(&buf, 256 + b_rope + b_qr + b_sc) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+    if (!device_alloc(&buf, 256 + b_rope + b_qr + b_sc)) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
     int32_t *np = (int32_t *)buf;
     float2 *rope = (float2 *)(buf + 256);
     int rc = 0;
@@ -2718,7 +2731,7 @@ extern "C" int xjh_sample(const float *logits, int n, int T, float temperature, 
         if (rand30[t] >= (1u << 30)) { snprintf(err, errlen, "sample: random number %u not below 2^30", rand30[t]); return -1; }
     const int prow = sample_part_rows(n), np = (n + prow - 1) / prow;
     uint32_t *d = nullptr;
-    if (hipMalloc(&d, 8 * (size_t)T + 8 * (size_t)T * np) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+    if (!device_alloc(&d, 8 * (size_t)T + 8 * (size_t)T * np)) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
     int32_t *o = (int32_t *)(d + T);
     unsigned long long *part = (unsigned long long *)(d + 2 * T);
     int rc = !draw || hipMemcpy(d, rand30, 4 * (size_t)T, hipMemcpyHostToDevice) == hipSuccess ? 0 : -1;
@@ -2736,7 +2749,7 @@ extern "C" int xjh_sample(const float *logits, int n, int T, float temperature, 
 extern "C" int xjh_argmax(const float *x, int n, int T, int32_t *out_host, char *err, size_t errlen) {
     if (!ops_stream()) return -1;
     int32_t *d = nullptr;
-    if (hipMalloc(&d, 4 * T) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+    if (!device_alloc(&d, 4 * T)) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
     int rc = argmax_rows_launch(x, n, T, d, g_stream) ? -1 : ops_done(err, errlen);
     if (!rc && hipMemcpy(out_host, d, 4 * T, hipMemcpyDeviceToHost) != hipSuccess) rc = -1;
     (void)hipFree(d);
@@ -2767,12 +2780,13 @@ extern "C" int xjh_delta_chunked(int H, int S, int T, int chunk, const float *q,
             if (g_work.p) (void)hipFree(g_work.p);
             g_work.p = nullptr;
             g_work.cap = 0;
-            if (hipMalloc(&g_work.p, wb) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+            if (!plain_alloc(&g_work.p, wb)) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
             g_work.cap = wb;
         }
         work = g_work.p;
     } else {
-        if (hipMalloc(&own, wb) != hipSuccess) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
+        if (lock.owns_lock()) lock.unlock();   // device_alloc may give the kept area back
+        if (!device_alloc(&own, wb)) { snprintf(err, errlen, "hipMalloc failed"); return -1; }
         work = own;
     }
     int rc = delta_chunked_launch(H, S, T, chunk, q, k, v, decay, beta, qscale, state, out, (float *)work, g_stream);

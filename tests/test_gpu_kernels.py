@@ -264,3 +264,35 @@ def test_delta_chunked_edges(S, T):
         oo[t] = np.einsum("hji,hi->hj", m, q[t]) * qs
     assert rel_l2(go, oo) < 5e-6
     assert rel_l2(gs, m) < 5e-6
+
+
+def test_delta_chunked_beyond_the_kept_area():
+    """A call whose work area exceeds the 512 MB that stay allocated between
+    calls takes one of its own: 7300 tokens of 32 heads of 128 (540 MB) in one
+    call and in two, cut at a chunk's edge with the state carried over, give
+    the same bits."""
+    T, H, S, cut = 7300, 32, 128, 3648
+    q, k, v, dec, beta = (np.tile(a, (T // 100,) + (1,) * (a.ndim - 1)) for a in _delta_inputs(100, H, S, 11))
+    st0 = np.zeros((H, S, S), np.float32)
+    go, gs = xp.delta(q, k, v, dec, beta, st0, 0.1, chunk=64)
+    o1, s1 = xp.delta(q[:cut], k[:cut], v[:cut], dec[:cut], beta[:cut], st0, 0.1, chunk=64)
+    o2, s2 = xp.delta(q[cut:], k[cut:], v[cut:], dec[cut:], beta[cut:], s1, 0.1, chunk=64)
+    assert np.array_equal(go[:cut].view(np.uint32), o1.view(np.uint32))
+    assert np.array_equal(go[cut:].view(np.uint32), o2.view(np.uint32))
+    assert np.array_equal(gs.view(np.uint32), s2.view(np.uint32))
+
+
+def test_failed_allocation_leaves_no_error():
+    """An allocation that cannot be met (1 PB) returns null, gives back the work
+    area kept by the chunked delta rule, and leaves no error for the launches
+    that follow to report: with an area kept and without."""
+    q, k, v, dec, beta = _delta_inputs(65, 4, 64, 12)
+    st0 = np.zeros((4, 64, 64), np.float32)
+    w = xp.DevWeight(xp.Q4_K, _weights(xp.Q4_K, 64, 256, 5), 64, 256)
+    xs = xp.fill_normal(40 * 256, 6, 1.0).reshape(40, 256)
+    want, _ = xp.delta(q, k, v, dec, beta, st0, 0.1, chunk=64)
+    y = xp.gemm(w, xs)
+    for _ in range(2):
+        assert not xp.lib().xjh_malloc(1 << 50)
+        assert np.array_equal(xp.gemm(w, xs), y)
+    assert np.array_equal(xp.delta(q, k, v, dec, beta, st0, 0.1, chunk=64)[0], want)
