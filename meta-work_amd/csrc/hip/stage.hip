@@ -2502,15 +2502,20 @@ static int gemm_enqueue(uint32_t type, const void *dw, int64_t n_rows, int64_t k
         cap = need;
         return true;
     };
+    auto zeros = [&](int32_t *&p, size_t &cap, size_t need) {   // zero once; the kernels leave them zero
+        if (need <= cap) return true;
+        if (!grow(p, cap, need)) return false;
+        if (hipMemsetAsync(p, 0, need * 4, st) == hipSuccess) return true;
+        cap = 0;
+        return false;
+    };
     if (T > gemm_max_tokens() && !((uintptr_t)x & 15)) {
         static uint8_t *wq = nullptr;
         static float *part = nullptr;
         static int32_t *cnt = nullptr;
         static size_t wq_cap = 0, part_cap = 0, cnt_cap = 0;
-        const size_t cneed = (size_t)wide_counters(n_rows, T);
-        const bool fresh = cneed > cnt_cap;   // zero once; the kernel leaves them zero
         if (!grow(wq, wq_cap, wide_wq_bytes((int)k, T)) || !grow(part, part_cap, (size_t)wide_part_floats(T)) ||
-            !grow(cnt, cnt_cap, cneed) || (fresh && hipMemsetAsync(cnt, 0, cneed * 4, st) != hipSuccess))
+            !zeros(cnt, cnt_cap, (size_t)wide_counters(n_rows, T)))
             return -1;
         WidePrep p{};
         p.x = x; p.xs = (int32_t)k; p.pro = PRO_NONE; p.wq = wq; p.K = (int32_t)k; p.T = T;
@@ -2532,11 +2537,9 @@ static int gemm_enqueue(uint32_t type, const void *dw, int64_t n_rows, int64_t k
     static int32_t *cnt = nullptr;
     static size_t xq_cap = 0, hq_cap = 0, part_cap = 0, cnt_cap = 0;
     const int64_t xs = xq_off((int)k).stride, hs = hq_stride((int)k);
-    const size_t need = (size_t)T * xs, hneed = (size_t)T * hs, pneed = (size_t)gemm_part_floats(n_rows, T),
-                 cneed = (size_t)gemm_counters(n_rows);
-    const bool fresh = cneed > cnt_cap;   // zero once; the kernel leaves them zero
-    if (!grow(xq, xq_cap, need) || !grow(hq, hq_cap, hneed) || !grow(part, part_cap, pneed) || !grow(cnt, cnt_cap, cneed) ||
-        (fresh && hipMemsetAsync(cnt, 0, cneed * 4, st) != hipSuccess))
+    const size_t need = (size_t)T * xs, hneed = (size_t)T * hs, pneed = (size_t)gemm_part_floats(n_rows, T);
+    if (!grow(xq, xq_cap, need) || !grow(hq, hq_cap, hneed) || !grow(part, part_cap, pneed) ||
+        !zeros(cnt, cnt_cap, (size_t)gemm_counters(n_rows)))
         return -1;
     GArgs p{};
     p.x = x; p.xs = (int32_t)k; p.pro = PRO_NONE; p.xq = xq; p.K = (int32_t)k; p.T = T; p.hq = hq;
