@@ -716,10 +716,11 @@ __device__ __forceinline__ void epi_load(const GSeg &sg, int64_t r, EpiIn<T> &e)
     // Unconditional loads at clamped in-row addresses (a loaded value that
     // reaches its register through a branch would make the first use of the
     // weight window wait for every outstanding load); values an epilogue does
-    // not use are ignored. y is valid memory for every epilogue.
+    // not use are ignored. y is valid memory for every epilogue (of a plain
+    // row its own element only: the one after the last row is not).
     const bool conv = sg.epi == EPI_CONV && sg.conv_k <= kConvPre;
-    const int KC = conv ? sg.conv_k : 2;
-    const float *ps = conv ? sg.conv_state + r * (KC - 1) : sg.y + r;
+    const int KC = conv ? sg.conv_k : 1;
+    const float *ps = conv ? sg.conv_state + r * (KC - 1) : sg.y + r + 1;   // (ps[-1], pw[0] read)
     const float *pw = conv ? sg.conv_w + r * KC : sg.y + r;
 #pragma unroll
     for (int t = 0; t < T; t++) e.y[t] = sg.y[(int64_t)t * sg.ys + r];
