@@ -78,10 +78,10 @@ __device__ __forceinline__ f4 mfma16(h8 a, h8 b, f4 c) { return __builtin_amdgcn
 
 // Lane l: 16 (4) bytes at p to LDS offset off + 16 l (4 l); off is uniform over the wavefront.
 __device__ __forceinline__ void dma16(const uint8_t *p, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(off) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(off) : "memory", "m0");
 }
 __device__ __forceinline__ void dma4(const uint8_t *p, uint32_t off) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(off) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(p), "s"(off) : "memory", "m0");
 }
 template <int N>
 __device__ __forceinline__ void wait_vm() {
