@@ -670,6 +670,7 @@ def test_sampler_nan_cases():
     assert orc.sample(lg, 0.0, 0) == 40
 
 
+@pytest.mark.skipif(not orc.ref_available(), reason="reference build (oracle/_ref) not present")
 def test_sampler_callback_draws_one_number_per_token(tiny_path):
     """The reference's own driver (xj_spec_next over oracle stages, k = 0) with
     the app's sample_cb over a stream of numbers: token g is the draw from the
