@@ -316,6 +316,13 @@ int xjh_gemv_noalloc(uint32_t type, const void *dw, int64_t n_rows, int64_t k, c
  * (src/xiaoju-pipe/metal/xj_kernels.metal:84-388) for long batches. */
 int xjh_gemm(uint32_t type, const void *dw, int64_t n_rows, int64_t k, const float *x, int T,
              float *y, int add, char *err, size_t errlen);
+/* Test hook, no counterpart in the reference: the GEMM of prompt pieces
+ * (33 <= T <= 1024) over nseg <= 4 matrices of one type that share the input x
+ * (16-byte aligned), y[i] of matrix i [T][n_rows[i]]; norm_w (may be NULL): x is
+ * RMS-normalised with it first (eps 1e-6). *kind: the kernel taken, 0 the one for
+ * up to 64 tokens, 1 slices of 64 tokens on it, 2 the one for more. */
+int xjh_gemm_piece(uint32_t type, const void *const *dw, const int64_t *n_rows, int nseg, int64_t k, const float *x,
+                   const float *norm_w, int T, float *const *y, int add, int *kind, char *err, size_t errlen);
 /* Mean ms of xjh_gemm (prep launch included) over rotating copies, like xjh_gemv_time. */
 double xjh_gemm_time(uint32_t type, void *const *dws, int n_copies, int64_t n_rows, int64_t k,
                      const float *x, int T, float *y, int iters, char *err, size_t errlen);

@@ -515,7 +515,8 @@ __global__ __launch_bounds__(kThreads, 2) void gemm_wide_kernel(const WideArgs a
 // L2. 64 tokens: 18432 x 2560 Q4_K 37.4 -> 28.0 us, 2560 x 4096 Q4_K 24.0 ->
 // 13.5, 2560 x 9216 Q6_K 37.3 -> 27.8, against 128-row groups whose weights
 // were decoded twice and whose K ranges met through HBM. Its error against
-// float64 is the smaller too (0.9..1.6e-7 against 1.0..2.4e-7: shorter sums).
+// float64 is no larger (Q4_K 2.4..3.1e-7 against 3.9..4.9e-7, Q6_K 0.9..1.3e-7
+// against 1.0..1.5e-7, inputs normal or heavy-tailed: shorter sums).
 // Below 33 tokens gemm.hip's kernels are as fast or faster (2560 x 9216 Q6_K at
 // 16: 15 against 20 us).
 template <bool Q6, int RT>
@@ -933,6 +934,14 @@ int wide_prep_launch(const WidePrep &in, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
+int gemm_wide_kind(const WideArgs &in) {
+    WideArgs a = in;
+    a.nb = a.K / 256;
+    int rows16 = 0;
+    for (int i = 0; i < a.nseg; i++) rows16 += (a.seg[i].N + 15) / 16;
+    return a.T <= kSkinnyT ? 0 : in_slices(a, rows16) ? 1 : 2;
+}
+
 int gemm_wide_launch(const WideArgs &in, int64_t part_floats, int n_cnt, hipStream_t st) {
     WideArgs a = in;
     if (!a.ss_n) a.ss_n = a.T;
@@ -947,9 +956,8 @@ int gemm_wide_launch(const WideArgs &in, int64_t part_floats, int n_cnt, hipStre
     }
     for (int i = a.nseg + 1; i <= kGemmMaxSeg; i++) a.rt0[i] = a.rt0[a.nseg];
     a.nb = a.K / 256;
-    int rows16 = 0;
-    for (int i = 0; i < a.nseg; i++) rows16 += (a.seg[i].N + 15) / 16;
-    if (a.T > kSkinnyT && in_slices(a, rows16)) {
+    const int kind = gemm_wide_kind(a);
+    if (kind == 1) {
         for (int t0 = 0; t0 < a.T; t0 += kSkinnyT) {
             WideArgs b = a;
             b.T = std::min(kSkinnyT, a.T - t0);
@@ -960,7 +968,7 @@ int gemm_wide_launch(const WideArgs &in, int64_t part_floats, int n_cnt, hipStre
         }
         return 0;
     }
-    if (a.T <= kSkinnyT) {
+    if (kind == 0) {
         const bool q6 = a.type == XJ_Q6_K;
         const int nt = a.T <= 48 ? 3 : 4;
         const SkPlan p = skinny_plan(q6, a.rt0[a.nseg], a.nb, nt);

@@ -204,6 +204,9 @@ size_t wide_wq_bytes(int K, int T);
 int64_t wide_part_floats(int T);
 int wide_counters(int64_t rows, int T);
 int wide_prep_launch(const WidePrep &a, hipStream_t st);
+// The kernel a launch takes: 0 the narrow one (up to 64 tokens), 1 slices of 64
+// tokens on it, 2 the wide one.
+int gemm_wide_kind(const WideArgs &a);
 int gemm_wide_launch(const WideArgs &a, int64_t part_floats, int n_cnt, hipStream_t st);
 
 // Repack a GGUF tensor into the device layout. dst must hold `bytes` =

@@ -2565,6 +2565,43 @@ extern "C" int xjh_gemm(uint32_t type, const void *dw, int64_t n_rows, int64_t k
     return ops_done(err, errlen);
 }
 
+extern "C" int xjh_gemm_piece(uint32_t type, const void *const *dw, const int64_t *n_rows, int nseg, int64_t k,
+                              const float *x, const float *norm_w, int T, float *const *y, int add, int *kind, char *err,
+                              size_t errlen) {
+    if (!ops_stream()) return -1;
+    int64_t rows = 0;
+    bool ok = (type == XJ_Q4_K || type == XJ_Q6_K) && T > gemm_max_tokens() && T <= kPieceT && k >= 256 && k % 256 == 0 &&
+              k <= (1 << 20) && nseg >= 1 && nseg <= kGemmMaxSeg && !(((uintptr_t)x | (uintptr_t)norm_w) & 15);
+    for (int i = 0; ok && i < nseg; i++) {
+        ok = n_rows[i] >= 1 && n_rows[i] <= (1 << 20);
+        rows += n_rows[i];
+    }
+    if (!ok) { snprintf(err, errlen, "unsupported GEMM shape/type"); return -1; }
+    WidePrep p{};
+    p.x = x; p.xs = (int32_t)k; p.pro = norm_w ? PRO_RMSU : PRO_NONE; p.pro_w = norm_w; p.K = (int32_t)k; p.T = T;
+    WideArgs g{};
+    g.type = type; g.K = (int32_t)k; g.T = T; g.nseg = nseg; g.eps = 1e-6f;
+    for (int i = 0; i < nseg; i++)
+        g.seg[i] = GemmSeg{(const uint8_t *)dw[i], (int32_t)n_rows[i], y[i], (int32_t)n_rows[i], add};
+    *kind = gemm_wide_kind(g);
+    const int64_t pf = wide_part_floats(T);
+    const int nc = wide_counters(rows, T);
+    int rc = -1;
+    if (device_alloc(&p.wq, wide_wq_bytes((int)k, T)) && device_alloc(&p.ss, 8 * (size_t)T * (k / 256)) &&
+        device_alloc(&g.part, 4 * (size_t)pf) && device_alloc(&g.cnt, 4 * (size_t)nc) &&
+        hipMemsetAsync(g.cnt, 0, 4 * (size_t)nc, g_stream) == hipSuccess) {
+        g.wq = p.wq;
+        g.ss = norm_w ? p.ss : nullptr;
+        if (!wide_prep_launch(p, g_stream) && !gemm_wide_launch(g, pf, nc, g_stream)) rc = ops_done(err, errlen);
+        else snprintf(err, errlen, "GEMM launch failed");
+    } else {
+        snprintf(err, errlen, "no memory for the GEMM's buffers");
+    }
+    (void)hipStreamSynchronize(g_stream);
+    for (void *b : {(void *)p.wq, (void *)p.ss, (void *)g.part, (void *)g.cnt}) if (b) (void)hipFree(b);
+    return rc;
+}
+
 extern "C" double xjh_gemm_time(uint32_t type, void *const *dws, int n_copies, int64_t n_rows, int64_t k, const float *x,
                                 int T, float *y, int iters, char *err, size_t errlen) {
     if (!ops_stream()) return -1;

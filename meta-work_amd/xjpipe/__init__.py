@@ -171,6 +171,7 @@ def lib():
     _sig(L, "xjh_gemv_noalloc", I, U32, P, I64, I64, P, I, P, I, CP, S)
     _sig(L, "xjh_gemm", I, U32, P, I64, I64, P, I, P, I, CP, S)
     _sig(L, "xjh_gemv_time", D, U32, C.POINTER(P), I, I64, I64, P, I, P, I, CP, S)
+    _sig(L, "xjh_gemm_piece", I, U32, C.POINTER(P), C.POINTER(I64), I, I64, P, P, I, C.POINTER(P), I, C.POINTER(I), CP, S)
     _sig(L, "xjh_gemm_time", D, U32, C.POINTER(P), I, I64, I64, P, I, P, I, CP, S)
     _sig(L, "xjh_norm", I, I, P, P, I, I, F, P, CP, S)
     _sig(L, "xjh_argmax", I, P, I, I, P, CP, S)
@@ -579,6 +580,22 @@ def gemm(w, x, add_to=None):
     err = _err()
     _check(lib().xjh_gemm(w.t, w.ptr, w.rows, w.k, dx.ptr, T, dy.ptr, int(add_to is not None), err, ERR), err, "gemm")
     return dy.get(np.float32, (T, w.rows))
+
+
+def gemm_piece(weights, x, norm_w=None, add_to=None):
+    """The GEMM of prompt pieces over matrices that share x [T][k] (xjh_gemm_piece, T > 32):
+    the outputs [T][rows] and the kernel taken (0 narrow, 1 slices on it, 2 wide)."""
+    x = np.ascontiguousarray(x, np.float32)
+    T, k = x.shape
+    n = len(weights)
+    dx, dn = Dev(x), Dev(np.ascontiguousarray(norm_w, np.float32)) if norm_w is not None else None
+    dy = [Dev(np.ascontiguousarray(a, np.float32)) for a in add_to] if add_to else [Dev(nbytes=T * w.rows * 4) for w in weights]
+    kind, err = C.c_int(-1), _err()
+    _check(lib().xjh_gemm_piece(weights[0].t, (C.c_void_p * n)(*[w.ptr for w in weights]),
+                                (C.c_int64 * n)(*[w.rows for w in weights]), n, k, dx.ptr, dn.ptr if dn else None, T,
+                                (C.c_void_p * n)(*[d.ptr for d in dy]), int(bool(add_to)), C.byref(kind), err, ERR),
+           err, "gemm piece")
+    return [d.get(np.float32, (T, w.rows)) for d, w in zip(dy, weights)], kind.value
 
 
 def gemm_time(weights, x, iters):
