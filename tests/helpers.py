@@ -1,7 +1,21 @@
 """Shared input builders for the tests and the golden-vector script."""
+import os
+import subprocess
+import sys
+import textwrap
+
 import numpy as np
 
 import xjpipe as xp
+
+
+def in_child(code, **env):
+    """Runs `code` in a python of its own, with switches the library reads once per process."""
+    path = os.pathsep.join(p for p in sys.path if p)
+    r = subprocess.run([sys.executable, "-c", textwrap.dedent(code)], env=dict(os.environ, PYTHONPATH=path, **env),
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stdout + r.stderr
+
 
 # fp16 bit patterns for block scales: zero, subnormals, smallest normal, +-1, +-65504, others
 EDGE_F16 = [0x0000, 0x0001, 0x03FF, 0x0400, 0x3C00, 0xBC00, 0x7BFF, 0xFBFF, 0x1234, 0x2E66, 0x8001, 0x5640]

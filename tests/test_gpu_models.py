@@ -16,6 +16,7 @@ import pytest
 
 import xjpipe as xp
 from conftest import GOLDEN
+from helpers import in_child
 
 pytestmark = pytest.mark.gpu
 
@@ -37,9 +38,9 @@ def first_divergence(a, b):
 
 @pytest.mark.parametrize("max_batch", [8, 64])
 def test_0_8b_greedy_256_steps(max_batch):
-    """max_batch 8 (the recorded runs' chunking: prefill on the GEMV) and 64
-    (prefill chunks on the matrix-core GEMM and the chunked delta rule); the
-    reference's tokens do not depend on the chunking."""
+    """The prompt as one piece on the matrix-core GEMM, attention and the
+    chunked delta rule, over stages of max_batch 8 and 64; the reference's
+    tokens do not depend on the chunking."""
     rec = fixture("greedy_0_8b.json")
     path = xp.cached_model(xp.CONFIG_0_8B, "synth08b")
     check_model(path, rec)
@@ -57,10 +58,31 @@ def test_0_8b_greedy_256_steps(max_batch):
     st.destroy()
 
 
+@pytest.mark.parametrize("name,n_gen", [("0_8b", 256), ("4b", 128)])
+def test_greedy_after_prefill_on_the_gemv(name, n_gen):
+    """The recorded runs' own chunking: the prompt in chunks of 8 on the GEMV and
+    the step kernels (XJ_PREFILL_GEMM=0), one stage whose layers run in parts."""
+    rec = fixture(f"greedy_{name}.json")
+    cfg, key = (xp.CONFIG_0_8B, "synth08b") if name == "0_8b" else (xp.CONFIG_4B, "synth4b")
+    path = xp.cached_model(cfg, key)
+    check_model(path, rec)
+    in_child(f"""
+        import numpy as np, xjpipe as xp
+        m = xp.Model({path!r})
+        ids = np.random.default_rng({rec["prompt_seed"]}).integers(0, m.hp.n_vocab, {rec["n_prompt"]}).astype(np.int32)
+        st = xp.HipStage(m, 0, m.hp.n_layer, {rec["n_ctx"]}, 8, True)
+        ch = xp.Chain([st])
+        toks = np.concatenate([ch.eval(ids), ch.decode({n_gen} - 1)]).tolist()
+        want = {rec["oracle_kvf16"]["tokens"][:n_gen]!r}
+        assert toks == want, next(i for i in range({n_gen}) if toks[i] != want[i])
+        ch.free()
+        st.destroy()
+        """, XJ_PREFILL_GEMM="0")
+
+
 @pytest.mark.parametrize("max_batch", [8, 64])
 def test_4b_two_stage_greedy_512_steps(max_batch):
-    """As the 0.8B test: prefill chunks of 8 (GEMV) and of 64 (matrix-core GEMM,
-    chunked delta rule)."""
+    """As the 0.8B test, over two stages."""
     rec = fixture("greedy_4b.json")
     path = xp.cached_model(xp.CONFIG_4B, "synth4b")
     check_model(path, rec)

@@ -6,10 +6,6 @@ prefill 12 tokens then 3 single tokens, head top-1, keep/rollback equal to
 never having computed the rolled-back tokens; plus greedy token identity.
 """
 import ctypes as C
-import os
-import subprocess
-import sys
-import textwrap
 
 import numpy as np
 import pytest
@@ -17,6 +13,7 @@ import pytest
 import oracle as orc
 import xjpipe as xp
 from conftest import rel_l2
+from helpers import in_child
 
 pytestmark = pytest.mark.gpu
 
@@ -28,14 +25,6 @@ def tiny(tiny_path):
 
 def embed(m, toks):
     return np.stack([orc.embed(m.ptr, int(t)) for t in toks]).astype(np.float32)
-
-
-def in_child(code, **env):
-    """Runs `code` in a python of its own, with switches the library reads once per process."""
-    path = os.pathsep.join(p for p in sys.path if p)
-    r = subprocess.run([sys.executable, "-c", textwrap.dedent(code)], env=dict(os.environ, PYTHONPATH=path, **env),
-                       capture_output=True, text=True, timeout=100)
-    assert r.returncode == 0, r.stdout + r.stderr
 
 
 def prompt_ids(m, n, seed):
@@ -195,14 +184,13 @@ def test_chain_split_and_vtable_agree(tiny):
 
 @pytest.mark.parametrize("cuts", [(0, 4, 8), (0, 2, 5, 8)])
 def test_pipelined_chain_prefill_equals_one_stage(tiny, cuts):
-    """A prompt of many chunks through a chain whose stages run on their own
-    streams, chunk k + 1 in stage i while chunk k is in stage i + 1
-    (xj_net.c:561-604): the logits of the last rows, the hidden rows left for
-    the drivers and the tokens decoded after it equal those of one stage
-    computing the same chunks in order, bit for bit."""
+    """A prompt beyond max_batch through a chain whose stages run on their own
+    streams (xj_net.c:561-604), here as one piece handed from stage to stage:
+    the logits of the last rows, the hidden rows left for the drivers and the
+    tokens decoded after it equal those of one stage, bit for bit."""
     m, L = tiny, tiny.hp.n_layer
     assert cuts[-1] == L
-    prompt = prompt_ids(m, 70, 29)            # max_batch 16: chunks 16 x 4 + 6
+    prompt = prompt_ids(m, 70, 29)            # max_batch 16: one piece of 70
     one = xp.HipStage(m, 0, L, 128, 16, True)
     c1 = xp.Chain([one])
     am1, lg1 = c1.eval(prompt, nlog=3, want_logits=True)
@@ -223,6 +211,61 @@ def test_pipelined_chain_prefill_equals_one_stage(tiny, cuts):
         c.free()
     for st in [one] + sts:
         st.destroy()
+
+
+@pytest.mark.parametrize("cuts", [(0, 4, 8), (0, 2, 5, 8)])
+def test_pipelined_pieces_equal_one_stage(tiny, cuts):
+    """2600 tokens: pieces of 1024, 1024 and 552, piece k + 1 in stage i while
+    piece k is in stage i + 1, so that a stage's buffer is overwritten only once
+    the next stage has taken it: the logits of the last rows and the tokens
+    decoded after them equal those of one stage, bit for bit, twice in a row."""
+    m, L = tiny, tiny.hp.n_layer
+    prompt = prompt_ids(m, 2600, 31)
+    one = xp.HipStage(m, 0, L, 2688, 16, True)
+    c1 = xp.Chain([one])
+    am1, lg1 = c1.eval(prompt, nlog=8, want_logits=True)   # the last chunk of max_batch holds 8 rows
+    t1 = c1.decode(12).tolist()
+    sts = [xp.HipStage(m, cuts[i], cuts[i + 1], 2688, 16, i + 2 == len(cuts)) for i in range(len(cuts) - 1)]
+    c2 = xp.Chain(sts)
+    for _ in range(2):
+        c2.reset()
+        am2, lg2 = c2.eval(prompt, nlog=8, want_logits=True)
+        assert np.array_equal(lg1.view(np.uint32), lg2.view(np.uint32))
+        assert am1.tolist() == am2.tolist()
+        assert c2.decode(12).tolist() == t1
+    for c in (c1, c2):
+        c.free()
+    for st in [one] + sts:
+        st.destroy()
+
+
+@pytest.mark.parametrize("cuts", [(0, 4, 8), (0, 2, 5, 8)])
+def test_pipelined_chunks_equal_one_stage(tiny_path, cuts):
+    """The same in chunks of max_batch (XJ_PREFILL_GEMM=0: no pieces): 70 tokens
+    in chunks of 16 x 4 + 6 through two and three stages, against one stage whose
+    layers run undivided (XJ_STAGE_SPLIT=1), bit for bit."""
+    in_child(f"""
+        import numpy as np, xjpipe as xp
+        m = xp.Model({tiny_path!r})
+        L, cuts = m.hp.n_layer, {cuts!r}
+        ids = np.random.default_rng(29).integers(0, m.hp.n_vocab, 70).astype(np.int32)
+        one = xp.HipStage(m, 0, L, 128, 16, True)
+        c1 = xp.Chain([one])
+        am1, lg1 = c1.eval(ids, nlog=3, want_logits=True)
+        t1 = c1.decode(12).tolist()
+        sts = [xp.HipStage(m, cuts[i], cuts[i + 1], 128, 16, i + 2 == len(cuts)) for i in range(len(cuts) - 1)]
+        c2 = xp.Chain(sts)
+        for _ in range(2):
+            c2.reset()
+            am2, lg2 = c2.eval(ids, nlog=3, want_logits=True)
+            assert np.array_equal(lg1.view(np.uint32), lg2.view(np.uint32))
+            assert am1.tolist() == am2.tolist()
+            assert c2.decode(12).tolist() == t1
+        for o in (c1, c2):
+            o.free()
+        for o in [one] + sts:
+            o.destroy()
+        """, XJ_PREFILL_GEMM="0", XJ_STAGE_SPLIT="1")
 
 
 def test_chain_verify_and_rollback(tiny):
