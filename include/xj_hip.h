@@ -164,8 +164,10 @@ typedef struct xjh_chain xjh_chain;
  * of eval_once (xj_net.c:541-559) with embedding and argmax on the device. */
 xjh_chain *xjh_chain_new(xj_stage **stages, int n_stages, char *err, size_t errlen);
 void       xjh_chain_free(xjh_chain *c);
-/* Feed n tokens in chunks of max_batch. When nlog > 0 the logits of the last
- * min(nlog, rows) rows of the final chunk are computed: copied to `logits`
+/* Feed n tokens: up to max_batch in one chunk, more in pieces of up to 1024
+ * tokens or in chunks of max_batch (xj_hip_stage_state_bytes). When nlog > 0 the
+ * logits of the last min(nlog, rows) rows, rows being what chunks of max_batch
+ * leave for the last one, are computed: copied to `logits`
  * [nlog][n_vocab] when it is not NULL, and their greedy argmax (first maximum)
  * written to `argmax`. keep != 0 turns this call into a verify (xj_net.c:668):
  * all n tokens in one chunk, recurrent checkpoints kept for rollback. The

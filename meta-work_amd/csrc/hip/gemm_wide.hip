@@ -1,7 +1,8 @@
 // Dequant-GEMM for prompt chunks and pieces of 33 tokens and more on the matrix cores
 // (gfx950): the products of gemm.hip (y[t][r] = sum_k deq(W_r)[k] x[t][k],
 // src/xiaoju-pipe/core/xj_cpu.c:36-54) for hundreds of tokens per launch, so
-// that a weight is decoded once per 128 tokens and wavefront pair.
+// that a weight is read once per 128 tokens and decoded once per 64 (by each of
+// the two wavefronts that share its rows).
 //
 // What bounds it: two f16 MFMAs per product (Q6_K: three), i.e. the matrix
 // cores; the weights' bytes are read once per token group through the caches.

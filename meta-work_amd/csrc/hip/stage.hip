@@ -108,7 +108,7 @@ struct HStage {
     int64_t gpart_floats = 0;
     int32_t *gcnt = nullptr;   // the GEMM's arrival counters (zero between launches)
     int32_t n_gcnt = 0;
-    WideBuf wide;              // buffers of the wide GEMM (max_batch > 64)
+    WideBuf wide;              // buffers of gemm_wide.hip (max_batch > 32)
     bool pieces = false;       // scratch for prompt pieces (twin_new)
     float2 *rope = nullptr;
     float *h_x = nullptr;            // pinned staging [max_batch][n_embd]
@@ -382,10 +382,10 @@ struct Gemv {
         const bool rms = a.pro == PRO_RMSU;
         if (!w && rms && rms_scale_launch(a.xq, xs, a.K, T, a.eps, tsc, st)) return -1;
         const int mt = gemm_max_tokens(), tile = gemv_max_tile(a.K);
-        // the Q4_K and Q6_K segments in one launch sharing the activations,
-        // each type on its own share of the work-groups (an attention
-        // layer's q|k and v: 20 us less per chunk than a launch of its own
-        // for v); XJ_GEMM_MIXED=0: one launch per type
+        // up to 32 tokens the Q4_K and Q6_K segments go in one launch sharing
+        // the activations, each type on its own share of the work-groups (an
+        // attention layer's q|k and v: 20 us less per chunk than a launch of its
+        // own for v); XJ_GEMM_MIXED=0: one launch per type, as wide_gemm has it
         static const bool mixed_on = env_int("XJ_GEMM_MIXED", 1) != 0;
         auto launch_tokens = [&](const GemmArgs &g) {
             for (int t0 = 0; t0 < T; t0 += mt) {
@@ -1235,7 +1235,8 @@ extern "C" int xj_hip_stage_restore(xj_stage *s, int slot, int n_past, char *err
 // ================================================================= chain ==
 
 // Tokens of a prompt that go through a layer at once, whatever max_batch is:
-// a weight is decoded once per 128 tokens, and every launch fills the chip.
+// a weight is read once per 128 tokens and decoded once per 64, and every launch
+// fills the chip.
 // Stages whose max_batch is above half of it run their own chunks.
 constexpr int kPieceT = 1024;
 constexpr int kMaxParts = 4;   // parts of a single stage's layers in a pipelined prefill
